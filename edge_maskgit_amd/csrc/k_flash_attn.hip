@@ -23,6 +23,7 @@
 // LDS rows are padded (K: D+8 halves, V^T: 72 halves) so the fragment reads are
 // bank-conflict free.
 #include <algorithm>
+#include <type_traits>
 
 #include "mgh_common.h"
 #include "mgh_kernels.h"
@@ -520,6 +521,440 @@ hipError_t launch_head(const FaArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Long sequences (S > 272): online softmax over 64-key chunks, a wave holding QT 16-query tiles
+// (each K / V fragment read from LDS serves QT tiles), QG waves side by side along the queries
+// and KS key groups of QG waves that take every KS-th chunk; the key groups' (max, sum, O) are
+// merged through LDS at the end. The work is VALU-bound (4.5 operations per score, one of them
+// a quarter-rate exp2), so:
+//  * the products, the P = hi + lo split, the row sums from the matrix unit and the transposed
+//    P . V are k_attn_head's; one 32-deep MFMA covers 32 features / keys, whose order inside a
+//    fragment is free as long as both operands share it, so K rows (padded with zeros to 32) and
+//    V^T rows (keys permuted within 32: position 8 lg + 4 (t % 2) + r holds key 16 (t % 2) + 4 lg
+//    + r) are read with one conflict-free 16-byte read per fragment;
+//  * the softmax reference of a query only has to be near its maximum: it starts 7 below the
+//    first chunk's (log2 units), so p = 2^7 there, and moves (and O is rescaled) only when a score
+//    of the wave exceeds it by more than 15, a wave-uniform branch almost never taken after the
+//    first chunk. p <= 2^15 is inside fp16, and the larger p keeps the lo parts of the small ones
+//    above the fp16 subnormals: with p <= 1, a row whose maximum stands 8 above its other scores
+//    lost 4.5e-6 of its weights' sum to them;
+//  * P . V and the row sums of a chunk start from zero and are added to O in fp32: the matrix
+//    unit's own accumulation over the whole sequence had twice the error against 64 bits
+//    (6.4e-7 against 3.3e-7 at S = 4097) for 6% less time;
+//  * keys past S are masked in the last chunk only.
+// K and V arrive as fp32: each workgroup loads the next chunk into registers (16-byte loads)
+// while it computes the current one, rounds once and stores fp16 to the other LDS buffer, V as
+// 4 x 4 blocks transposed in registers: one barrier per chunk.
+// A sequence of 2^k + 1 tokens (the class token) leaves one query past the whole blocks: a last
+// block with a single wave's queries is split over the keys instead, each wave reading its own
+// fragments from memory without the staging or its barriers.
+// Measured (16 heads, D = 48, one image) against the kernel for any strides: S = 1025 114 -> 18 us,
+// S = 4097 549 -> 121 us (16-bit MFMA work at full rate: ~50 us, VALU ~55 us), error against
+// 64 bits 3.8e-7 -> 2.3e-7 and 6.6e-7 -> 2.9e-7.
+constexpr int LKT = 64;                  // keys per chunk
+constexpr int LVLD = LKT + 8;            // V^T row stride (halves): 9 16-byte slots
+template <int DC>
+constexpr int kLongKLD = DC <= 2 ? 40 : 72;   // K row stride (halves): 32 or 64 features + 8
+
+template <int DC, int QG, int QT, int KS, bool I16>
+__global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull, int heads) {
+    constexpr int D = 16 * DC, KLD = kLongKLD<DC>, KC = (DC + 1) / 2, NW = QG * KS;
+    constexpr int GT = 64 * QG;          // threads per key group
+    constexpr int KV4 = LKT * D / 4;     // 16-byte pieces of a chunk's K
+    constexpr int UK = (KV4 + GT - 1) / GT, VB = LKT / 4 * (D / 4), UV = (VB + GT - 1) / GT;
+    constexpr int CH = LKT * KLD + D * LVLD;     // halves per chunk buffer
+    constexpr int MR = QT * (4 * DC + 2);   // floats a lane hands over in the merge
+    constexpr int STAGE = 2 * KS * CH * 2, MERGE = NW * 64 * MR * 4;
+    __shared__ __attribute__((aligned(16))) char lds[STAGE > MERGE ? STAGE : MERGE];
+
+    const int S = a.S;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = wave / QG, qg = wave - kg * QG, gt = tid - kg * GT;
+    const int l16 = lane & 15, lg = lane >> 4;
+    // whole blocks first, each XCD taking contiguous runs of (head, block) so that its L2 holds
+    // few heads' K and V; then the heads' partial blocks
+    const int nf = nfull * heads;
+    int hb, qb;
+    if ((int)blockIdx.x < nf) {
+        const int lid = xcd_remap(blockIdx.x, nf);
+        hb = lid / nfull, qb = lid - hb * nfull;
+    } else {
+        hb = blockIdx.x - nf, qb = nfull;
+    }
+    const int h = hb % a.H, b = hb / a.H;
+    const int64_t base = (int64_t)b * a.st[3] + (int64_t)h * a.st[2];
+    const int q0b = qb * 16 * QT * QG;
+    // a partial block with one wave's queries: its waves split the keys
+    const bool split = NW > 1 && S - q0b <= 16 * QT;
+    const int q0 = q0b + (split ? 0 : 16 * QT * qg);
+    const bool active = q0 < S;
+
+    // staging: this key group's chunk c, K pieces (key, 4 features) and V blocks (4 keys x 4
+    // features; lanes run over 4 feature blocks, then key blocks: 64-byte row segments). Buffer
+    // loads over the head's rows: loop-invariant lane offsets, the chunk in the scalar offset,
+    // rows past S outside the range (zeros), so the loop spends no vector instruction on
+    // addresses or bounds.
+    constexpr int EB = I16 ? 2 : 4;      // bytes per element
+    typedef std::conditional_t<I16, f16x4, f32x4> E4;
+    const uint32_t ext = (uint32_t)(((int64_t)(S - 1) * a.st[1] + D) * EB);
+    auto rsrc = [&](const float* p, const _Float16* p16) {
+        void* q = I16 ? (void*)(p16 + base) : (void*)(p + base);
+        return __builtin_amdgcn_make_buffer_rsrc(q, (short)0, (int)ext, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rsk = rsrc(a.k, a.k16), rsv = rsrc(a.v, a.v16);
+    auto ld4 = [](__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t so) -> E4 {
+        if constexpr (I16) return __builtin_bit_cast(E4, __builtin_amdgcn_raw_buffer_load_b64(r, (int)vo, (int)so, 0));
+        else return __builtin_bit_cast(E4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)vo, (int)so, 0));
+    };
+    auto h4 = [](E4 v) { return f16x4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]}; };
+    const uint32_t rowb = (uint32_t)a.st[1] * EB;
+    uint32_t ok[UK], ov[UV], sk[UK], sv[UV];     // byte offsets in the source, half offsets in LDS
+#pragma unroll
+    for (int u = 0; u < UK; u++) {
+        const int i = gt + GT * u, key = i / (D / 4), d = 4 * (i - key * (D / 4));
+        ok[u] = key * rowb + EB * d;
+        sk[u] = key * KLD + d;
+    }
+#pragma unroll
+    for (int u = 0; u < UV; u++) {
+        const int i = gt + GT * u, kb = (i >> 2) & 15, db = (i & 3) + 4 * (i >> 6);
+        ov[u] = 4 * kb * rowb + EB * 4 * db;
+        sv[u] = LKT * KLD + 4 * db * LVLD + 32 * (kb >> 3) + 8 * (kb & 3) + 4 * ((kb >> 2) & 1);
+    }
+    E4 rk[UK], rv[UV][4];
+    auto load = [&](int c) {
+        const uint32_t so = (uint32_t)c * LKT * rowb;
+#pragma unroll
+        for (int u = 0; u < UK; u++)
+            if (KV4 % GT == 0 || gt + GT * u < KV4)
+                rk[u] = ld4(rsk, ok[u], so);
+#pragma unroll
+        for (int u = 0; u < UV; u++)
+            if (VB % GT == 0 || gt + GT * u < VB)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    rv[u][j] = ld4(rsv, ov[u], so + j * rowb);
+    };
+    auto store = [&](int buf) {
+        _Float16* B = (_Float16*)lds + (buf * KS + kg) * CH;
+#pragma unroll
+        for (int u = 0; u < UK; u++)
+            if (KV4 % GT == 0 || gt + GT * u < KV4)
+                *(f16x4*)(B + sk[u]) = h4(rk[u]);
+#pragma unroll
+        for (int u = 0; u < UV; u++)
+            if (VB % GT == 0 || gt + GT * u < VB)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    *(f16x4*)(B + sv[u] + e * LVLD) =
+                        f16x4{(_Float16)rv[u][0][e], (_Float16)rv[u][1][e], (_Float16)rv[u][2][e], (_Float16)rv[u][3][e]};
+    };
+
+    // Q as the B operand: lane = query 16 qt + l16, features 32 c + 8 lg + j (zeros past D)
+    f16x8 qf[QT][KC];
+#pragma unroll
+    for (int qt = 0; qt < QT; qt++) {
+        const int qi = min(q0 + 16 * qt + l16, S - 1);
+        const int64_t qrow = base + (int64_t)qi * a.st[1];
+#pragma unroll
+        for (int c = 0; c < KC; c++) {
+            const int d = 32 * c + 8 * lg;
+            qf[qt][c] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            if (d < D) qf[qt][c] = load_h8<I16, false>(a.q, a.q16, qrow + d);
+        }
+    }
+    // the features between D and the padded width meet zeros of Q: they only have to be finite
+    if (D % 32) {
+        for (int i = tid; i < 2 * KS * LKT; i += 64 * NW)
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                *(f16x8*)((_Float16*)lds + (i / LKT) * CH + (i % LKT) * KLD + D + 8 * e) = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+
+    const float scale2 = a.scale * 1.4426950408889634f;
+    const float m1 = opaque_neg_one();
+    const f16x8 ones = {1, 1, 1, 1, 1, 1, 1, 1};
+    // softmax reference (scaled, log2 units), O^T (register r of chunk c: feature 16 c + 4 lg + r of
+    // query l16) and the row sums (every register of S1)
+    float mref[QT], S1[QT];
+    f32x4 O[QT][DC];
+#pragma unroll
+    for (int qt = 0; qt < QT; qt++) {
+        mref[qt] = -1e30f;
+        S1[qt] = 0.f;
+#pragma unroll
+        for (int c = 0; c < DC; c++) O[qt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    // NT key tiles from key0 on: kfrag(t, i) is the K fragment of tile t, features 32 i + 8 lg + j;
+    // vfrag(p, c) the V^T fragment of tiles 2p, 2p + 1, feature 16 c + l16. (MASK is a property
+    // of the call, not a branch between the score MFMAs and their use: around such a branch the
+    // compiler left out the wait for the MFMA results.)
+    auto compute = [&](auto ntc, auto mask, int key0, auto kfrag, auto vfrag) {
+        constexpr int NT = decltype(ntc)::value;
+        f32x4 sc[QT][NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            f16x8 kf[KC];
+#pragma unroll
+            for (int i = 0; i < KC; i++) kf[i] = kfrag(t, i);
+#pragma unroll
+            for (int qt = 0; qt < QT; qt++) {
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < KC; i++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[i], qf[qt][i], acc, 0, 0, 0);
+                sc[qt][t] = acc;
+            }
+        }
+        if (decltype(mask)::value) {             // keys past S
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (key0 + 16 * t + 4 * lg + r >= S)
+#pragma unroll
+                        for (int qt = 0; qt < QT; qt++) sc[qt][t][r] = -INFINITY;
+        }
+        float mx[QT];
+        bool up = false;
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++) {
+            float v = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                v = fmaxf(fmaxf(v, sc[qt][t][0]), sc[qt][t][1]);
+                v = fmaxf(fmaxf(v, sc[qt][t][2]), sc[qt][t][3]);
+            }
+            mx[qt] = v * scale2;
+            up = up || mx[qt] > mref[qt] + 15.f;
+        }
+        if (__any(up)) {
+#pragma unroll
+            for (int qt = 0; qt < QT; qt++) {
+                float v = fmaxf(mx[qt] - 7.f, mref[qt]);
+                v = fmaxf(v, __shfl_xor(v, 16));
+                v = fmaxf(v, __shfl_xor(v, 32));
+                const float al = __builtin_amdgcn_exp2f(mref[qt] - v);
+                mref[qt] = v;
+                S1[qt] *= al;
+#pragma unroll
+                for (int cc = 0; cc < DC; cc++) O[qt][cc] *= al;
+            }
+        }
+        f32x4 sc1[QT], oc[QT][DC];
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++) {
+            sc1[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int cc = 0; cc < DC; cc++) oc[qt][cc] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int p = 0; p < NT / 2; p++) {
+            f16x8 vf[DC];
+#pragma unroll
+            for (int cc = 0; cc < DC; cc++) vf[cc] = vfrag(p, cc);
+#pragma unroll
+            for (int qt = 0; qt < QT; qt++) {
+                float e[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    e[j] = __builtin_amdgcn_exp2f(fmaf(sc[qt][2 * p + j / 4][j % 4], scale2, -mref[qt]));
+                u32x4 hi, lo;
+                auto u = [](auto v) { return __builtin_bit_cast(uint32_t, v); };
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const auto hh = __builtin_amdgcn_cvt_pkrtz(e[2 * j], e[2 * j + 1]);
+                    hi[j] = u(hh);
+                    lo[j] = u(__builtin_amdgcn_cvt_pkrtz(fmaf((float)hh[0], m1, e[2 * j]), fmaf((float)hh[1], m1, e[2 * j + 1])));
+                }
+                const f16x8 ph = __builtin_bit_cast(f16x8, hi), pl = __builtin_bit_cast(f16x8, lo);
+#pragma unroll
+                for (int cc = 0; cc < DC; cc++) {
+                    oc[qt][cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[cc], pl, oc[qt][cc], 0, 0, 0);
+                    oc[qt][cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[cc], ph, oc[qt][cc], 0, 0, 0);
+                }
+                sc1[qt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pl, sc1[qt], 0, 0, 0);
+                sc1[qt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, ph, sc1[qt], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++) {
+            S1[qt] += sc1[qt][0];
+#pragma unroll
+            for (int cc = 0; cc < DC; cc++) O[qt][cc] += oc[qt][cc];
+        }
+    };
+
+    if (!split) {
+        // chunks it * KS + kg; the last round, which holds the sequence's last chunk, masks
+        const int nch = (S + LKT - 1) / LKT, nit = (nch + KS - 1) / KS;
+        auto step = [&](auto mask, int buf, int c) {
+            const _Float16* Ks = (const _Float16*)lds + (buf * KS + kg) * CH;
+            const _Float16* Vt = Ks + LKT * KLD;
+            compute(std::integral_constant<int, LKT / 16>{}, mask, c * LKT,
+                    [&](int t, int i) { return *(const f16x8*)&Ks[(16 * t + l16) * KLD + 32 * i + 8 * lg]; },
+                    [&](int p, int cc) { return *(const f16x8*)&Vt[(16 * cc + l16) * LVLD + 32 * p + 8 * lg]; });
+        };
+        load(kg);
+        store(0);
+        for (int it = 0; it + 1 < nit; it++) {
+            __syncthreads();             // this buffer is filled, the other one no longer read
+            load((it + 1) * KS + kg);
+            if (active) step(std::false_type{}, it & 1, it * KS + kg);
+            store((it + 1) & 1);
+        }
+        __syncthreads();
+        const int c = (nit - 1) * KS + kg;
+        if (active && c < nch) step(std::true_type{}, (nit - 1) & 1, c);
+    } else {
+        // 32-key groups wave, wave + NW, ..., each wave's fragments straight from memory (rows
+        // past S and features past D outside the buffer range: zeros). Holding the next group's
+        // values as well would cost the registers that let this block share a CU with two whole
+        // ones
+        const int ng = (S + 31) / 32;
+        E4 kr[2][KC][2];
+        std::conditional_t<I16, _Float16, float> vr[DC][8];
+        auto fetch = [&](int g) {
+            const uint32_t so = 32u * g * rowb;
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < KC; i++) {
+                    const int d = 32 * i + 8 * lg;
+                    const uint32_t o = d < D ? (16 * t + l16) * rowb + EB * d : 0x80000000u;
+                    kr[t][i][0] = ld4(rsk, o, so);
+                    kr[t][i][1] = ld4(rsk, o + 4 * EB, so);
+                }
+#pragma unroll
+            for (int cc = 0; cc < DC; cc++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int o = (int)((16 * (j >> 2) + 4 * lg + (j & 3)) * rowb + EB * (16 * cc + l16));
+                    if constexpr (I16)
+                        vr[cc][j] = __builtin_bit_cast(_Float16, __builtin_amdgcn_raw_buffer_load_b16(rsv, o, (int)so, 0));
+                    else
+                        vr[cc][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsv, o, (int)so, 0));
+                }
+        };
+        for (int g = wave; g < ng; g += NW) {
+            fetch(g);
+            f16x8 kf[2][KC], vf[DC];
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < KC; i++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) kf[t][i][j] = (_Float16)kr[t][i][j >> 2][j & 3];
+#pragma unroll
+            for (int cc = 0; cc < DC; cc++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) vf[cc][j] = (_Float16)vr[cc][j];
+            compute(std::integral_constant<int, 2>{}, std::true_type{}, 32 * g, [&](int t, int i) { return kf[t][i]; },
+                    [&](int, int cc) { return vf[cc]; });
+        }
+    }
+
+    // merge: the waves that share queries (the key groups; with split, all waves) hand their
+    // (reference, sum, O) to the first of them
+    if (KS > 1 || split) {
+        __syncthreads();
+        float* mg = (float*)lds;         // [wave][MR][64 lanes]
+        const bool first = kg == 0 && (!split || qg == 0);
+        if (!first && active) {
+            float* w = mg + wave * MR * 64 + lane;
+#pragma unroll
+            for (int qt = 0; qt < QT; qt++) {
+                w[(qt * (4 * DC + 2)) * 64] = mref[qt];
+                w[(qt * (4 * DC + 2) + 1) * 64] = S1[qt];
+#pragma unroll
+                for (int c = 0; c < DC; c++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) w[(qt * (4 * DC + 2) + 2 + 4 * c + r) * 64] = O[qt][c][r];
+            }
+        }
+        __syncthreads();
+        if (!first) return;
+        const int step = split ? 1 : QG;
+        for (int o = wave + step; o < NW; o += step) {
+            const float* w = mg + o * MR * 64 + lane;
+#pragma unroll
+            for (int qt = 0; qt < QT; qt++) {
+                const float mo = w[(qt * (4 * DC + 2)) * 64], mn = fmaxf(mref[qt], mo);
+                const float al = __builtin_amdgcn_exp2f(mref[qt] - mn), be = __builtin_amdgcn_exp2f(mo - mn);
+                mref[qt] = mn;
+                S1[qt] = fmaf(w[(qt * (4 * DC + 2) + 1) * 64], be, S1[qt] * al);
+#pragma unroll
+                for (int c = 0; c < DC; c++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        O[qt][c][r] = fmaf(w[(qt * (4 * DC + 2) + 2 + 4 * c + r) * 64], be, O[qt][c][r] * al);
+            }
+        }
+    }
+    if (!active) return;
+    const bool vec = a.os[0] == 1 && ((a.os[1] | a.os[2] | a.os[3]) & 3) == 0 &&
+                     ((uintptr_t)(a.o16 ? (const void*)a.o16 : (const void*)a.o) & 15) == 0;
+#pragma unroll
+    for (int qt = 0; qt < QT; qt++) {
+        const float inv = 1.f / S1[qt];
+        const int qi = q0 + 16 * qt + l16;
+        if (qi >= S) continue;
+        const int64_t ro = (int64_t)b * a.os[3] + (int64_t)h * a.os[2] + (int64_t)qi * a.os[1];
+#pragma unroll
+        for (int c = 0; c < DC; c++) {
+            const int d = 16 * c + 4 * lg;
+            f32x4 v = O[qt][c] * inv;
+            // (rounded to fp32 before the fp16 store rounds again: kept from fusing into one step)
+            asm volatile("" : "+v"(v));
+            if (vec) {
+                if (a.o16)
+                    *(f16x4*)(a.o16 + ro + d) = f16x4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+                else
+                    *(f32x4*)(a.o + ro + d) = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int64_t e = ro + (int64_t)(d + r) * a.os[0];
+                    if (a.o16) a.o16[e] = (_Float16)v[r];
+                    else a.o[e] = v[r];
+                }
+            }
+        }
+    }
+}
+
+template <int DC, int QG, int QT, int KS>
+void launch_long_t(const FaArgs& a, hipStream_t s) {
+    const int qb = 16 * QT * QG, nfull = a.S / qb, heads = a.H * a.B;
+    const dim3 grid((unsigned)(heads * (nfull + (a.S % qb ? 1 : 0)))), block(64 * QG * KS);
+    if (a.q16) hipLaunchKernelGGL((k_attn_long<DC, QG, QT, KS, true>), grid, block, 0, s, a, nfull, heads);
+    else hipLaunchKernelGGL((k_attn_long<DC, QG, QT, KS, false>), grid, block, 0, s, a, nfull, heads);
+}
+
+// Few query blocks (one image of up to ~1500 tokens): 64 queries and two key groups per workgroup,
+// so that every CU has a workgroup of eight waves; from about 200 128-query blocks (120 at D = 64,
+// whose 64-query form holds 150 registers) 128 queries per workgroup, each K / V fragment serving
+// two query tiles. Measured, 16 heads, D = 48, fp32 q/k/v, (64 queries x 2 key groups) against 128
+// queries: S = 600 10.0 / 15.4 us, 1025 18.0 / 23.3, 2049 48.9 / 45.3, 4097 156 / 124, S = 1025
+// with 4 images 45.7 / 37.9; D = 64: S = 1500, 12 heads 36.9 / 33.3. One key group with 64
+// queries lies between the two everywhere but within 10% of the better one.
+template <int DC>
+hipError_t launch_long(const FaArgs& a, hipStream_t s) {
+    const int64_t nb = (int64_t)a.H * a.B * ((a.S + 127) / 128);
+    if (nb < (DC <= 3 ? 200 : 120)) launch_long_t<DC, 4, 1, 2>(a, s);
+    else launch_long_t<DC, 4, 2, 1>(a, s);
+    return hipGetLastError();
+}
+
+// q/k/v whose rows are features in order, spaced at least a head apart, that the staging's 8- or
+// 16-byte loads and 31-bit byte offsets can take; the workgroup count fits an int
+bool long_ok(const FaArgs& a, int D) {
+    auto al = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
+    const bool ptrs = a.q16 ? al(a.q16) && al(a.k16) && al(a.v16) : al(a.q) && al(a.k) && al(a.v);
+    return D % 16 == 0 && ptrs && a.st[0] == 1 && a.st[1] >= D && ((int64_t)a.S + 512) * a.st[1] * 4 < (1ll << 31) &&
+           a.st[1] % 4 == 0 && a.st[2] % 4 == 0 && a.st[3] % 4 == 0 && a.scale > 0.f &&
+           (int64_t)a.H * a.B * (a.S / 32 + 1) < (1ll << 31);
+}
+
 bool head_ok(const FaArgs& a, int D) {
     auto al = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
     const bool ptrs = a.q16 ? al(a.q16) && al(a.k16) && al(a.v16) : al(a.q) && al(a.k) && al(a.v);
@@ -531,8 +966,23 @@ bool head_ok(const FaArgs& a, int D) {
 
 hipError_t launch_flash_attn_f16kv(const FaArgs& a, int D, hipStream_t s) {
     if (a.S <= 0 || a.H <= 0 || a.B <= 0) return hipSuccess;
-    if (a.q16 && !head_ok(a, D)) return hipErrorInvalidValue;   // fp16 inputs: whole-head kernel only
-    if (head_ok(a, D)) {
+    const bool head = head_ok(a, D);
+    if (a.q16 && !head) return hipErrorInvalidValue;   // fp16 inputs: S <= 512 with aligned rows only
+    // The whole-head kernel up to 17 key tiles (S = 272, one 256-token image and its class token:
+    // 16 images 13.0 against 14.6 us for the long kernel, one image 6.3 against 6.6, fp16 q/k/v);
+    // beyond, its score registers leave one or two waves per SIMD and the long kernel wins (one
+    // image, S = 512: 10.2 against 8.0 us; 4 images, S = 400: 26.2 against 11.8). Both input
+    // types take the same kernel, so their results stay equal.
+    if ((!head || a.S > 272) && long_ok(a, D)) {
+        switch (D) {
+            case 16: return launch_long<1>(a, s);
+            case 32: return launch_long<2>(a, s);
+            case 48: return launch_long<3>(a, s);
+            case 64: return launch_long<4>(a, s);
+            default: break;
+        }
+    }
+    if (head) {
         switch (D) {
             case 16: return launch_head<1>(a, s);
             case 32: return launch_head<2>(a, s);
@@ -541,6 +991,7 @@ hipError_t launch_flash_attn_f16kv(const FaArgs& a, int D, hipStream_t s) {
             default: break;
         }
     }
+    // any strides
     const dim3 grid((unsigned)((a.S + 63) / 64), (unsigned)a.H, (unsigned)a.B), block(256);
     switch (D) {
         case 16: hipLaunchKernelGGL(k_flash_attn_f16kv<1>, grid, block, 0, s, a); break;

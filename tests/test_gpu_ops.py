@@ -114,7 +114,7 @@ def _qkv(rng, D, S, H, B):
     return [rng.standard_normal(shape).astype(np.float32) for _ in range(3)]
 
 
-# S <= 512 runs the whole-head kernel (K/V of a head resident in LDS), longer sequences the
+# S <= 272 runs the whole-head kernel (K/V of a head resident in LDS), longer sequences the
 # chunked online-softmax kernel
 @pytest.mark.parametrize("D,S,H,B", [(48, 1, 2, 1), (48, 16, 2, 1), (48, 17, 2, 1), (48, 64, 3, 2), (48, 65, 2, 1),
                                      (48, 257, 16, 2), (64, 130, 4, 1), (16, 40, 1, 1), (32, 300, 2, 1),
@@ -181,8 +181,73 @@ def test_flash_attn_o16_is_rounded_output(ctx, S):
     assert np.array_equal(h.view(np.uint16), o.astype(np.float16).view(np.uint16))
 
 
+# The long kernel (S > 272) at the edges of its blocks and chunks: a whole number of 64-key chunks
+# and one key past it; a last block of one query (split over the keys), of exactly one wave's
+# queries and one more; the 64-query form with two key groups (an odd and an even number of
+# chunks) and, from 200 (D = 64: 120) 128-query blocks, the 128-query form; padded rows (q/k/v
+# strides 4 elements past the heads); fp16 output; outputs whose rows are not 16-byte aligned.
+@pytest.mark.parametrize("D,S,H,B,pad,opad", [
+    (48, 273, 3, 1, 0, 0), (48, 576, 2, 1, 0, 0), (48, 577, 2, 1, 4, 0), (48, 592, 2, 2, 0, 0), (48, 593, 2, 1, 0, 1),
+    (16, 300, 2, 1, 4, 0), (32, 385, 3, 2, 0, 2), (64, 641, 2, 1, 0, 0), (64, 384, 40, 1, 0, 0), (64, 1025, 14, 1, 4, 1),
+    (48, 385, 50, 1, 0, 0), (48, 400, 25, 2, 4, 0), (48, 417, 50, 1, 0, 3), (32, 2049, 12, 1, 0, 0), (16, 513, 40, 1, 0, 0)])
+def test_flash_attn_long(ctx, D, S, H, B, pad, opad):
+    """against float64 on the fp16-rounded operands: |o - ref| <= 2e-5 max|ref|, the bar of the
+    other attention kernels (fp32 sums over S / 64 chunks: about 1e-6)"""
+    print(f"flash_attn_long D={D} S={S} H={H} B={B} pad={pad} opad={opad}", flush=True)
+    rng = np.random.default_rng(11 * D + S + H)
+    E = H * D
+    R, RO = 3 * E + pad, E + opad
+    wide = rng.standard_normal((B, S, R)).astype(np.float32)
+    # scores that grow along the keys move the softmax reference many times
+    wide[:, :, E:2 * E] *= np.linspace(0.2, 4.0, S)[None, :, None]
+    h = wide[:, :, :3 * E].astype(np.float16).astype(np.float64).reshape(B, S, 3, H, D)
+    scale = D ** -0.5
+    ref = np.empty((B, S, H, D))
+    for b in range(B):
+        for i in range(H):
+            s = h[b, :, 0, i] @ h[b, :, 1, i].T * scale
+            p = np.exp(s - s.max(-1, keepdims=True))
+            ref[b, :, i] = p @ h[b, :, 2, i] / p.sum(-1, keepdims=True)
+    ref = ref.reshape(B * S, E)
+    dw, do, dh = ctx.upload(wide), ctx.alloc(B * S * RO * 4), ctx.alloc(B * S * RO * 2)
+    st, ost = (1, R, D, R * S), (1, RO, D, RO * S)
+    ctx.flash_attn_f16kv(dw.ptr, dw.ptr + 4 * E, dw.ptr + 8 * E, st, D, S, H, B, scale, do, o_strides=ost)
+    ctx.flash_attn_f16kv_o16(dw.ptr, dw.ptr + 4 * E, dw.ptr + 8 * E, st, D, S, H, B, scale, dh, o_strides=ost)
+    o = ctx.download(do, (B * S, RO), np.float32)[:, :E]
+    o16 = ctx.download(dh, (B * S, RO), np.float16)[:, :E]
+    for t in (dw, do, dh):
+        ctx.free(t)
+    err = _rel(o, ref)
+    print(f"  rel err {err:.2e}")
+    assert err <= 2e-5
+    assert np.array_equal(o16.view(np.uint16), o.astype(np.float16).view(np.uint16))
+
+
+def test_flash_attn_long_strides(ctx):
+    """The same attention through strides the long kernel does not take (features two elements
+    apart: the kernel for any strides) and through ones it takes: both within 2e-5 max|ref| of
+    each other."""
+    D, S, H, B = 48, 600, 3, 2
+    E = H * D
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((3, B * S, E)).astype(np.float32)
+    two = np.zeros((3, B * S, 2 * E), np.float32)
+    two[:, :, ::2] = x
+    outs = []
+    for a, m in ((x, 1), (two, 2)):
+        d = [ctx.upload(a[i]) for i in range(3)]
+        do = ctx.alloc(B * S * E * 4)
+        st = (m, m * E, m * D, m * E * S)
+        ctx.flash_attn_f16kv(d[0], d[1], d[2], st, D, S, H, B, 0.144, do, o_strides=(1, E, D, E * S))
+        outs.append(ctx.download(do, (B * S, E), np.float32))
+        for t in d + [do]:
+            ctx.free(t)
+    assert _rel(outs[0], outs[1]) <= 2e-5
+
+
 @pytest.mark.parametrize("D,S,H,B,pad", [(48, 257, 16, 2, 0), (48, 1, 2, 1, 0), (64, 130, 4, 1, 0), (32, 512, 2, 1, 0),
-                                         (48, 257, 4, 2, 4), (16, 33, 1, 3, 4), (64, 512, 2, 1, 12)])
+                                         (48, 257, 4, 2, 4), (16, 33, 1, 3, 4), (64, 512, 2, 1, 12),
+                                         (48, 273, 3, 1, 4), (48, 385, 50, 1, 0), (16, 300, 1, 1, 12)])
 def test_flash_attn_f16in_equals_rounded_inputs(ctx, D, S, H, B, pad):
     """The fp16-input variant on q/k/v rounded to fp16 gives the same bits as the fp32-input
     attention (which rounds its inputs to fp16 on load), for both output types, with q/k/v
