@@ -31,7 +31,7 @@ HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
 
 KERNEL_SOURCES = ["k_quant_act.hip", "k_gemm_i8.hip",
                   "k_pack_w.hip", "k_gemm_qp.hip", "k_layernorm.hip", "k_flash_attn.hip",
-                  "k_gemm_f32.hip", "k_glue.hip", "k_ops.hip", "k_vqgan.hip", "k_conv_i8.hip", "noalloc.hip", "k_decode.hip", "k_gemm_fc.hip", "mgh_api.cpp"]
+                  "k_gemm_f32.hip", "k_glue.hip", "k_ops.hip", "k_vqgan.hip", "k_conv_split.hip", "k_conv_i8.hip", "noalloc.hip", "k_decode.hip", "k_gemm_fc.hip", "mgh_api.cpp"]
 # Per-source extra flags. Every MFMA kernel keeps its MFMA results in VGPRs: the int8 GEMMs'
 # per-block scale arithmetic then reads them without v_accvgpr_read copies, and in the
 # unrolled K loops of the FC GEMM and the attention's tile loops the accumulators no longer
@@ -40,7 +40,7 @@ KERNEL_SOURCES = ["k_quant_act.hip", "k_gemm_i8.hip",
 # occupancy and fewer registers.
 _VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 EXTRA_FLAGS = {src: _VGPR_FORM for src in ("k_gemm_i8.hip", "k_gemm_qp.hip", "k_conv_i8.hip", "k_gemm_fc.hip",
-                                           "k_flash_attn.hip", "k_gemm_f32.hip", "k_vqgan.hip")}
+                                           "k_flash_attn.hip", "k_gemm_f32.hip", "k_vqgan.hip", "k_conv_split.hip")}
 # C++ host runtime (graph API mirror, GGUF loader, transformer builder, HipRuntime, mgr C ABI):
 # plain host code over the libmgh C ABI, compiled with g++ into lib/libmg_hip.so.
 HOST_SOURCES = ["mg-tensor.cpp", "mg-model.cpp", "mg-transformer.cpp", "mg-vqgan.cpp", "mg-hip.cpp", "mgr_api.cpp"]

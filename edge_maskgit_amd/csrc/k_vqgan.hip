@@ -43,6 +43,8 @@ constexpr int CBM = 64, CBN = 64, CBK = 16, CPAD = 4;
 // ---- packed-weight implicit GEMM (IC % 16 == 0): K in tap-major order k = (kh*KW + kw)*IC + ic,
 // so a 16-wide K slab is one tap and 16 consecutive input channels: the im2col gather needs one
 // bounds check per pixel and slab, and its loads step through channel planes.
+// For IC % 32 == 0 (every decoder conv) launch_conv_split takes the wide form; this kernel keeps the
+// other multiples of 16 and images of 2 GiB and more.
 constexpr int PBM = 128, PBN = 128, PBK = 16, PST = PBK + 4;   // LDS rows padded to 20 floats
 
 // SPLIT: blockIdx.z = image * splits + split; the split's K range [split*kps, +kps) is summed
@@ -616,7 +618,8 @@ ConvPkPlan conv_pk_plan(int M, int OC, int K) {
     const int slabs = K / PBK;
     const int want = (int)std::min<int64_t>((512 + tiles - 1) / tiles, slabs / 9);
     if (tiles >= 384 || want < 2) return p;
-    const int per = (slabs + want - 1) / want;
+    int per = (slabs + want - 1) / want;
+    if (K % 32 == 0 && !conv_pk_narrow(OC)) per = (per + 1) & ~1;   // whole 32-deep steps (launch_conv_split)
     p.kps = per * PBK;
     p.splits = (slabs + per - 1) / per;
     return p;
@@ -652,6 +655,7 @@ hipError_t launch_conv2d_pk(const ConvPkArgs& a0, float* ws, hipStream_t s) {
     if (p.splits == 1) {
         const dim3 grid(gx, gy, (unsigned)a.N);
         if (nar) hipLaunchKernelGGL(k_conv2d_pkn<false>, grid, block, 0, s, a);
+        else if (conv_split_ok(a)) launch_conv_split(a, s);
         else hipLaunchKernelGGL(k_conv2d_pk<false>, grid, block, 0, s, a);
         return hipGetLastError();
     }
@@ -665,6 +669,7 @@ hipError_t launch_conv2d_pk(const ConvPkArgs& a0, float* ws, hipStream_t s) {
         a.N = g;
         const dim3 grid(gx, gy, (unsigned)(g * p.splits));
         if (nar) hipLaunchKernelGGL(k_conv2d_pkn<true>, grid, block, 0, s, a);
+        else if (conv_split_ok(a) && a.kps % 32 == 0) launch_conv_split(a, s);
         else hipLaunchKernelGGL(k_conv2d_pk<true>, grid, block, 0, s, a);
         const int64_t total = (int64_t)g * out_img;
         const int64_t nb = std::min<int64_t>((total + 255) / 256, 8192);

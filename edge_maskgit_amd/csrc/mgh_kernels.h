@@ -240,6 +240,9 @@ struct ConvPkPlan {
     int splits, kps;       // K split into `splits` ranges of kps values (a multiple of 16)
 };
 bool conv_pk_narrow(int OC);
+// the same on the bf16 matrix unit (k_conv_split.hip; a.splits and a.kps set, kps % 32 == 0)
+bool conv_split_ok(const ConvPkArgs& a);
+void launch_conv_split(const ConvPkArgs& a, hipStream_t s);
 ConvPkPlan conv_pk_plan(int M, int OC, int K);   // per image: independent of the batch
 size_t conv_pk_ws_bytes(int M, int OC, int N, int K);    // split-K partials, 0 without a split
 hipError_t launch_conv_pack(const float* ker, float* wpk, int IC, int taps, int OC, hipStream_t s);

@@ -33,9 +33,10 @@ def ctx():
     c.close()
 
 
-# kernels: IC % 16 == 0 packed tap-major MFMA ("pk": 128 x 128 tiles, "pkn": 256 x 16 for
-# OC <= 16; split over K when one image's output gives too few workgroups); else OC <= 8 one
-# thread per pixel ("few"), or the reference-layout MFMA ("gen")
+# kernels: IC % 16 == 0 packed tap-major MFMA ("pk": OC > 16, with IC % 32 == 0 on three bf16 parts
+# per value, else on fp32 MFMA; "pkn": 256 x 16 for OC <= 16; split over K when one image's output
+# gives too few workgroups); else OC <= 8 one thread per pixel ("few"), or the reference-layout
+# MFMA ("gen")
 CONV = [  # IW, IH, IC, N, KW, KH, OC, stride, pad
     (9, 7, 5, 2, 3, 3, 7, 1, 1), (10, 10, 3, 1, 3, 3, 8, 2, 1), (5, 5, 2, 1, 5, 5, 3, 1, 2),
     (7, 7, 4, 1, 3, 3, 3, 1, 0), (32, 32, 128, 1, 3, 3, 3, 1, 1),                     # few, pkn
@@ -47,6 +48,9 @@ CONV = [  # IW, IH, IC, N, KW, KH, OC, stride, pad
     (128, 128, 128, 1, 3, 3, 128, 1, 1), (32, 32, 256, 1, 1, 1, 256, 1, 0),           # pk
     (11, 6, 16, 1, 5, 5, 24, 1, 2),                                                   # pk, 5x5
     (256, 192, 16, 1, 3, 3, 16, 1, 1),                                                # pk, no split
+    (16, 15, 32, 1, 1, 1, 17, 1, 0), (17, 15, 64, 3, 3, 3, 129, 1, 1),      # pk: one step; tile edges
+    (67, 61, 96, 1, 3, 3, 127, 1, 1), (33, 65, 160, 4, 5, 3, 40, 2, 2),     # 3 and 5 steps per tap
+    (257, 200, 32, 1, 3, 3, 64, 1, 1), (240, 221, 64, 1, 1, 1, 128, 1, 0),  # 256-pixel tiles, ragged
     (4, 4, 4096, 260, 3, 3, 16, 1, 1),            # pk, 256 splits: images launched in groups of 255 + 5
 ]
 
@@ -127,6 +131,53 @@ def test_conv2d_ex_bias_residual_packed(ctx, IW, IH, IC, N, KW, KH, OC, stride, 
         ctx.free(dP)
     for b in (dX, dK, dB, dR, dY):
         ctx.free(b)
+
+
+def test_conv2d_not_finite(ctx):
+    """infinities, NaN and values next to the largest float in the input and the weights give what
+    fp32 products and sums give, with 128- and 256-pixel tiles and with K split"""
+    for IW, IC, OC, N in ((24, 64, 20, 1), (128, 32, 130, 1), (16, 512, 128, 8)):
+        print(f"conv2d not finite IW={IW} IC={IC} OC={OC} N={N}", flush=True)
+        rng = np.random.default_rng(IW)
+        x = rng.standard_normal((N, IC, IW, IW)).astype(np.float32)
+        ker = rng.standard_normal((OC, IC, 3, 3)).astype(np.float32) / 8
+        x[0, 3, 4, 5], x[0, 1, 9, 1], x[-1, 2, 12, 13] = np.inf, np.nan, -np.inf
+        x[0, 7, 13, 3] = np.finfo(np.float32).max
+        ker[5, 3], ker[6, 2, 0, 0] = 0.0, np.inf
+        dX, dK, dY = ctx.upload(x), ctx.upload(ker), ctx.alloc(N * OC * IW * IW * 4)
+        ctx.conv2d(dX, IW, IW, IC, N, dK, 3, 3, OC, 1, 1, dY)
+        y = ctx.download(dY, (N, OC, IW, IW), np.float32)
+        for b in (dX, dK, dY):
+            ctx.free(b)
+        # class of every output: what the values that are not finite reach (a zero weight times an
+        # infinity is NaN); the finite rest against float64
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = np.zeros((N, OC, IW, IW))
+            xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (1, 1), (1, 1)))
+            k64 = ker.astype(np.float64)
+            for kh in range(3):
+                for kw in range(3):
+                    win = xp[:, :, kh:kh + IW, kw:kw + IW].reshape(N, IC, -1)
+                    for n in range(N):
+                        fin = np.where(np.isfinite(win[n]), win[n], 0.0)
+                        kfin = np.where(np.isfinite(k64[:, :, kh, kw]), k64[:, :, kh, kw], 0.0)
+                        s = kfin @ fin
+                        for c, p in zip(*np.nonzero(~np.isfinite(win[n]))):
+                            s[:, p] += k64[:, c, kh, kw] * win[n, c, p]
+                        s[6] += k64[6, 2, kh, kw] * win[n, 2] if not np.isfinite(k64[6, 2, kh, kw]) else 0.0
+                        want[n] += s.reshape(OC, IW, IW)
+        # (an infinite weight over padding is not a product: those taps are skipped)
+        edge = np.zeros((IW, IW), bool)
+        edge[0, :] = edge[:, 0] = True
+        with np.errstate(invalid="ignore", over="ignore"):
+            w32 = want.astype(np.float32)
+        chk = np.ones_like(w32, bool)
+        chk[:, 6, edge] = False
+        assert np.array_equal(np.isnan(y[chk]), np.isnan(w32[chk]))
+        inf = np.isinf(w32) & chk
+        assert np.array_equal(y[inf], w32[inf])
+        ok = np.isfinite(w32) & chk
+        assert (np.abs(y[ok] - w32[ok]) / np.maximum(1.0, np.abs(w32[ok]))).max() <= 2e-5
 
 
 # planes of 4k elements take the 16-byte path (9 x 7, 5 x 3: single elements); a group spans
