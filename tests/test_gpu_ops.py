@@ -326,6 +326,68 @@ def test_gemm_f32_vs_oracle(ctx, M, N, K, act, res):
     assert err <= 1e-5
 
 
+# Edges of the 64 x 64 tiles and of the 32-deep K steps, with up to one workgroup per CU (two LDS
+# buffers) and more (one buffer); operands over 12 decades, so that all three parts of a value and the
+# small products count.
+@pytest.mark.parametrize("M,N,K,act,res", [(1, 1, 32, 0, False), (63, 65, 64, 0, True), (64, 64, 96, 1, False),
+                                           (65, 63, 128, 2, True), (1088, 1024, 32, 0, False), (1089, 961, 96, 0, True),
+                                           (1100, 1000, 160, 1, False)])
+def test_gemm_f32_vs_float64(ctx, M, N, K, act, res):
+    """each output within 2e-6 of sum_k |w x| + |bias| + |resid|, a few fp32 roundings of the running
+    sum (2^-24 each, at most six per 32 values of k: below 3e-7 sqrt(6 K / 32))"""
+    print(f"gemm_f32 float64 M={M} N={N} K={K} act={act} resid={res}", flush=True)
+    rng = np.random.default_rng(M + 3 * N + K)
+
+    def wide(*shape):
+        return (rng.standard_normal(shape) * 10.0 ** rng.uniform(-6, 6, shape)).astype(np.float32)
+
+    w, x = wide(N, K), wide(M, K)
+    bias, resid = wide(N), wide(M, N) if res else None
+    dW, dX, dB, dY = ctx.upload(w), ctx.upload(x), ctx.upload(bias), ctx.alloc(M * N * 4)
+    dR = ctx.upload(resid) if res else None
+    ctx.gemm_f32(dW, N, K, dX, M, dB, act, dR, dY)
+    y = ctx.download(dY, (M, N), np.float32)
+    for t in (dW, dX, dB, dY, dR):
+        if t is not None:
+            ctx.free(t)
+    w, x, bias = w.astype(np.float64), x.astype(np.float64), bias.astype(np.float64)
+    ref, mag = x @ w.T + bias, np.abs(x) @ np.abs(w).T + np.abs(bias)
+    from scipy.special import erf
+    with np.errstate(over="ignore"):
+        ref = 0.5 * ref * (1 + erf(ref / np.sqrt(2))) if act == 1 else ref / (1 + np.exp(-ref)) if act == 2 else ref
+    if res:
+        ref, mag = ref + resid, mag + np.abs(resid)
+    err = float((np.abs(y - ref) / mag).max())
+    print(f"  err / sum of magnitudes {err:.2e}")
+    assert err <= 2e-6
+
+
+@pytest.mark.parametrize("M", [70, 1100])
+def test_gemm_f32_not_finite(ctx, M):
+    """infinities, NaN and values next to the largest float give what fp32 products and sums give"""
+    N, K = 1000, 64
+    print(f"gemm_f32 not finite M={M}", flush=True)
+    rng = np.random.default_rng(M)
+    w, x = (rng.standard_normal(s).astype(np.float32) for s in ((N, K), (M, K)))
+    x[3, 5], x[66, 9], x[M - 1, 0] = np.inf, np.nan, -np.inf
+    x[7] = 0
+    x[7, 2] = np.finfo(np.float32).max
+    w[11, 2], w[12, 5], w[13, 3], w[14] = 1.0, 0.0, np.inf, 0.0
+    dW, dX, dY = ctx.upload(w), ctx.upload(x), ctx.alloc(M * N * 4)
+    ctx.gemm_f32(dW, N, K, dX, M, None, 0, None, dY)
+    y = ctx.download(dY, (M, N), np.float32)
+    for t in (dW, dX, dY):
+        ctx.free(t)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = (x.astype(np.float64)[:, None, :] * w.astype(np.float64)[None]).sum(-1) if M < 100 else \
+            np.stack([(x[m].astype(np.float64) * w.astype(np.float64)).sum(-1) for m in range(M)])
+        ref = ref.astype(np.float32)
+    assert np.array_equal(np.isnan(y), np.isnan(ref))
+    assert np.array_equal(np.isinf(y), np.isinf(ref)) and np.array_equal(np.sign(y[np.isinf(y)]), np.sign(ref[np.isinf(ref)]))
+    ok = np.isfinite(ref)
+    assert np.abs(y[ok] / np.maximum(np.abs(ref[ok]), 1.0) - ref[ok] / np.maximum(np.abs(ref[ok]), 1.0)).max() <= 2e-5
+
+
 # ---- glue ------------------------------------------------------------------------------
 def test_get_rows_add_copy(ctx):
     print("glue ops", flush=True)
