@@ -268,6 +268,25 @@ __global__ __launch_bounds__(256) void k_pack_wdq(const uint8_t* __restrict__ w,
     }
 }
 
+// Q4_K in the K-loop-dequant layout -> fp16 [N][K], the values the K loop decodes (and k_pack_w16
+// stores): one thread per 8 values, eight lanes per row and 64-deep stage (128-byte row segments).
+// Bound by the fp16 it writes (768 x 3072: 4.7 MB, 2.6 us).
+__global__ __launch_bounds__(256) void k_expand_q4(const uint8_t* __restrict__ w, u32x4* __restrict__ out, int N, int K) {
+    const int S = K / 64;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;     // (group, stage, row, K half, slice)
+    const int64_t G = ((int64_t)N + 15) / 16, gs = i >> 7;
+    if (gs >= G * S) return;
+    const int64_t g = gs / S;
+    const int st = (int)(gs - g * S), r = (int)(i >> 3) & 15, h = (int)(i >> 2) & 1, q = (int)i & 3;
+    const int64_t n = 16 * g + r;
+    if (n >= N) return;
+    const uint32_t c = *(const uint32_t*)(w + gs * 512 + 256 * h + 64 * q + 4 * r);
+    const u32x4 hd = ((const u32x4*)(w + G * S * 512))[(g * (K / 256) + (st >> 2)) * 16 + r];
+    float s0, m0, s1, m1;
+    q4_scales(hd, st, s0, m0, s1, m1);
+    out[(n * K + 64 * st + 32 * h + 8 * q) / 8] = __builtin_bit_cast(u32x4, deq_q4v(c, h ? s1 : s0, h ? m1 : m0));
+}
+
 // The 32 values of block t of weight row n as the reference decodes them (fp32): Q8_0
 // d * q (DEQ_Q8, mg-opencl.cpp:386-387), Q4_K (d * sc) * q - dmin * m (deq_q4k_elem, :252-262;
 // the 6-bit scale / min unpacking of get_scale_min_k4, :178-184). Bytes are read one at a
@@ -1167,6 +1186,13 @@ hipError_t launch_pack_weights_dq(int wtype, const void* w, void* out, int N, in
         hipLaunchKernelGGL(k_pack_wdq<12>, grid, block, 0, s, (const uint8_t*)w, (uint8_t*)out, N, K);
     else
         return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+hipError_t launch_expand_q4(const void* wdq, void* out, int N, int K, hipStream_t s) {
+    const int64_t threads = ((int64_t)N + 15) / 16 * (K / 64) * 128;
+    if (threads == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_expand_q4, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, (const uint8_t*)wdq, (u32x4*)out, N, K);
     return hipGetLastError();
 }
 

@@ -936,6 +936,34 @@ int mgh_f32_to_f16(mgh_ctx* c, const float* x, int64_t n, void* x16) {
 
 namespace {
 
+// Decoding Q4_K in the K loop costs ~23 VALU per fragment in every activation tile; expanding the
+// weights to fp16 first costs a launch and their fp16 bytes (4-5 us) and lets the call run the
+// fp16 form's plans. Measured per FC, cold buffers, fp32 / fp16 activations, K loop against expanded:
+// M = 4097 QKV 46.0 / 32.5 against 39.2 / 30.2 us, out 22.2 / 20.5 against 16.3 / 13.9, up 52.5 / 44.0
+// against 48.1 / 41.8, down 72.8 / 51.5 against 45.3 / 38.0; M = 1025 QKV 19.2 / 15.6 against 17.7 /
+// 16.8, up 24.3 / 22.1 against 21.8 / 18.9; M = 700 QKV 15.3 / 13.0 against 17.4 / 14.1 but out 16.0 /
+// 9.9 against 10.5 / 9.1, down 25.6 / 24.1 against 23.9 / 21.7. Q8_0 decodes in 1.5 VALU per weight:
+// its K loop stays ahead.
+bool expand_pays(int M, int N) { return M >= (N <= 1024 ? 700 : 1024); }
+
+// Weights of a call on Q4_K bytes with many rows: expanded to fp16 in the context scratch (from `off`
+// on) and multiplied in that form. A call that cannot have the scratch (not while a graph is
+// captured, or the allocation fails) decodes in the K loop as before.
+void expand_weights(mgh_ctx* c, mgh::GemmH16Args& a, size_t off) {
+    if (a.wq != MGH_WTYPE_Q4_K || !expand_pays(a.M, a.N)) return;
+    const size_t need = off + (size_t)a.N * a.K * 2;
+    if (c->scratch_bytes < need && (c->capturing || (size_t)a.N * a.K * 2 > ((size_t)1 << 28))) return;
+    if (ensure_scratch(c, need) != MGH_OK) {
+        c->err.clear();
+        (void)hipGetLastError();
+        return;
+    }
+    char* w16 = (char*)c->scratch + off;
+    if (mgh::launch_expand_q4(a.w, w16, a.N, a.K, c->stream) != hipSuccess) return;
+    a.w = w16;
+    a.wq = 0;
+}
+
 // The dequantize-fused FC entry points, for either weight form: wq 0 (fp16 [N][K] from
 // mgh_pack_weights_f16) or 8 / 12 (the K-loop-dequant layout of mgh_pack_weights_dq).
 int gemm_h16_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, int K, const void* x16, int M,
@@ -948,6 +976,7 @@ int gemm_h16_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, int K
     a.x = (const _Float16*)x16; a.w = w; a.wq = wq;
     a.bias = bias; a.resid = resid; a.y = y16 ? nullptr : y; a.y16 = y16;
     a.M = M; a.N = N; a.K = K; a.act = act;
+    expand_weights(c, a, 0);
     return run_gemm_h16(c, a);
 }
 
@@ -974,7 +1003,9 @@ int gemm_h16_ln_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, in
     a.x = (const _Float16*)x16; a.w = w; a.wq = wq;
     a.bias = bias; a.resid = resid; a.y = y;
     a.M = M; a.N = N; a.K = K; a.act = act;
-    const mgh::H16Plan p = mgh::gemm_h16_plan(M, N, K, false, wq);
+    const size_t y_b = no_y ? round256((size_t)M * N * 4) : 0;
+    expand_weights(c, a, y_b);
+    const mgh::H16Plan p = mgh::gemm_h16_plan(M, N, K, false, a.wq);
     if (!mgh::use_gemv_h16(M, K) && p.splits > 1 && act == 0) {
         // the split-K reduce normalizes each row as it leaves: one launch fewer
         if (int r = ensure_qp_ws(c, p.ws_bytes)) return r;
@@ -985,7 +1016,8 @@ int gemm_h16_ln_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, in
         return MGH_OK;
     }
     if (no_y) {
-        if (int r = ensure_scratch(c, round256((size_t)M * N * 4))) return r;
+        // (expanded weights lie behind y: the scratch they are in already holds it)
+        if (int r = ensure_scratch(c, y_b)) return r;
         a.y = y = (float*)c->scratch;
     }
     if (int r = run_gemm_h16(c, a)) return r;
@@ -1014,11 +1046,15 @@ int gemm_h16_f32in_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N,
     a.w = w; a.wq = wq;
     a.bias = bias; a.resid = resid; a.y = y;
     a.M = M; a.N = N; a.K = K; a.act = act;
-    if (!round_act_pass(M, N)) {
+    const bool pass = round_act_pass(M, N);
+    const size_t x_b = pass ? round256((size_t)M * K * 2) : 0;
+    expand_weights(c, a, x_b);
+    if (!pass) {
         a.xf = x;                               // rounded while the GEMM reads them
     } else {
-        // a rounding pass, then the fp16-operand kernel and its tile plans
-        if (int r = ensure_scratch(c, round256((size_t)M * K * 2))) return r;
+        // a rounding pass, then the fp16-operand kernel and its tile plans (expanded weights lie
+        // behind the rounded rows: the scratch they are in already holds both)
+        if (int r = ensure_scratch(c, x_b)) return r;
         MGH_HIP(c, mgh::launch_f32_to_f16(x, (_Float16*)c->scratch, (int64_t)M * K, c->stream), "k_f32_to_f16");
         a.x = (const _Float16*)c->scratch;
     }

@@ -197,6 +197,8 @@ hipError_t launch_pack_weights_f16(int wtype, const void* w, void* out, int N, i
 hipError_t launch_dequant_weights_f32(int wtype, const void* w, float* out, int N, int K, hipStream_t s);
 size_t packed_weight_bytes_dq(int wtype, int64_t N, int64_t K);
 hipError_t launch_pack_weights_dq(int wtype, const void* w, void* out, int N, int K, hipStream_t s);
+// Q4_K in that layout -> fp16 [N][K] (16-byte aligned), the form of wq = 0
+hipError_t launch_expand_q4(const void* wdq, void* out, int N, int K, hipStream_t s);
 hipError_t launch_f32_to_f16(const float* x, _Float16* h, int64_t n, hipStream_t s);
 // ln: the split-K reduce also writes the LayerNorm-affine of y's rows (the plan must split K;
 // act 0, fp32 y, N % 256 == 0, N <= 2048). N <= kFcMaxN: the tiled epilogue addresses a tile's

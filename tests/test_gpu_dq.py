@@ -360,3 +360,69 @@ def test_dequant_weights_f32_matches_oracle(ctx, wtype, N, K):
     ctx.free(dO)
     want = oracle.dequant(wtype, wq, N, K)
     assert np.array_equal(got.view(np.uint32), want.astype(np.float32).view(np.uint32))
+
+
+# Q4_K calls with many rows (from 700 rows for N <= 1024, from 1024 for wider outputs) decode the
+# weights once into fp16 scratch: rows and columns off the tiles, a last 16-row weight group that is
+# not full, one super-block and several; at the rule's edges and with the rounding pass (its rows lie
+# before the weights in the scratch).
+@pytest.mark.parametrize("M,N,K", [(700, 100, 256), (703, 1020, 768), (1024, 1028, 512), (1030, 772, 1280),
+                                   (4100, 3076, 256)])
+def test_q4k_expanded_equals_fp16_copies(ctx, M, N, K):
+    """the same launches as on fp16 copies follow, so every output equals theirs bit for bit"""
+    print(f"q4k expanded M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    wq = oracle.quantize(ema.WTYPE_Q4_K, (rng.standard_normal((N, K)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    bias, resid = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    dW, dX, dX16 = ctx.upload(wq), ctx.upload(x), ctx.upload(x.astype(np.float16))
+    dB, dR = ctx.upload(bias), ctx.upload(resid)
+    dP, dQ = ctx.alloc(ema.packed_weight_bytes_f16(N, K)), ctx.alloc(ema.packed_weight_bytes_dq(ema.WTYPE_Q4_K, N, K))
+    ctx.pack_weights_f16(ema.WTYPE_Q4_K, dW, N, K, dP)
+    ctx.pack_weights_dq(ema.WTYPE_Q4_K, dW, N, K, dQ)
+    out = [ctx.alloc(M * N * 4) for _ in range(2)]
+
+    def same(f16, bytes_, dtype=np.float32):
+        f16(out[0])
+        bytes_(out[1])
+        a, b = (ctx.download(o, (M, N), dtype) for o in out)
+        assert np.isfinite(a.astype(np.float32)).all() and np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+    q = ema.WTYPE_Q4_K
+    same(lambda y: ctx.gemm_h16_f32in(dP, N, K, dX, M, dB, 1, dR, y), lambda y: ctx.gemm_dq_f32in(q, dQ, N, K, dX, M, dB, 1, dR, y))
+    same(lambda y: ctx.gemm_h16(dP, N, K, dX16, M, dB, 0, dR, y), lambda y: ctx.gemm_dq(q, dQ, N, K, dX16, M, dB, 0, dR, y))
+    same(lambda y: ctx.gemm_h16_y16(dP, N, K, dX16, M, dB, 2, None, y),
+         lambda y: ctx.gemm_dq_y16(q, dQ, N, K, dX16, M, dB, 2, None, y), np.float16)
+    for b in [dW, dX, dX16, dB, dR, dP, dQ] + out:
+        ctx.free(b)
+
+
+def test_q4k_expanded_ln_and_capture():
+    """the FC + LayerNorm call whose y lies in the scratch before the weights, and a call captured on a
+    context without scratch (decoded in the K loop: another summation order)"""
+    M, N, K = 1040, 768, 768
+    rng = np.random.default_rng(9)
+    wq = oracle.quantize(ema.WTYPE_Q4_K, (rng.standard_normal((N, K)) * 0.02).astype(np.float32))
+    x16, resid = rng.standard_normal((M, K)).astype(np.float16), rng.standard_normal((M, N)).astype(np.float32)
+    gamma, beta = (1 + 0.1 * rng.standard_normal(N)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    q = ema.WTYPE_Q4_K
+    with ema.Context(0) as c:
+        dW, dX, dR, dG, dE = c.upload(wq), c.upload(x16), c.upload(resid), c.upload(gamma), c.upload(beta)
+        dP, dQ = c.alloc(ema.packed_weight_bytes_f16(N, K)), c.alloc(ema.packed_weight_bytes_dq(q, N, K))
+        c.pack_weights_f16(q, dW, N, K, dP)
+        c.pack_weights_dq(q, dW, N, K, dQ)
+        y, ln, ln2 = c.alloc(M * N * 4), c.alloc(M * N * 4), c.alloc(M * N * 4)
+        c.graph_begin()
+        c.gemm_dq(q, dQ, N, K, dX, M, None, 0, dR, y)
+        g = c.graph_end()
+        for _ in range(3):
+            g.launch()
+            c.sync()
+            got = c.download(y, (M, N), np.float32)
+            c.gemm_h16(dP, N, K, dX, M, None, 0, dR, ln)
+            want = c.download(ln, (M, N), np.float32)
+            assert _rel(got, want) <= 1e-5
+        g.destroy()
+        c.gemm_h16_ln(dP, N, K, dX, M, None, 0, dR, None, dG, dE, 1e-12, ln)
+        c.gemm_dq_ln(q, dQ, N, K, dX, M, None, 0, dR, None, dG, dE, 1e-12, ln2)
+        assert np.array_equal(c.download(ln, (M, N), np.float32), c.download(ln2, (M, N), np.float32))
