@@ -13,7 +13,9 @@
 // rest LDS latency and VALU that the two waves per SIMD do not cover), error against 64 bits 3.1e-7
 // -> 2.7e-7. The small products in accumulators of their own: 1.1e-7 but 98 us (64 registers more,
 // so fragments are read just before use); the six of a step summed from zero: 7e-8 but 108 us (64
-// additions per step).
+// additions per step). With K split, where a workgroup per CU and its latency set the time, the
+// accumulators of their own cost nothing and are taken (128 x 128 x 128, two images: 66 us either way,
+// 7.9e-8 against 1.9e-7).
 //  * gather: a thread takes one pixel and 8 consecutive channels per piece as buffer loads (pixel
 //    offset per lane, channel plane in the scalar offset; a tap outside the image takes an offset
 //    past the range, which loads zero), one K step ahead in registers;
@@ -116,11 +118,16 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
         return Frag3{*(const bf16x8*)q, *(const bf16x8*)(q + part), *(const bf16x8*)(q + 2 * part)};
     };
 
-    f32x4 acc[J][I];
+    Frag3 fa[I], fb[2];
+    f32x4 acc[J][I], rest[SPLIT ? J : 1][I];
 #pragma unroll
     for (int j = 0; j < J; j++)
 #pragma unroll
-        for (int i = 0; i < I; i++) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < I; i++) acc[j][i] = rest[SPLIT ? j : 0][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto prod = [&](int i, int j, const Frag3& b) {
+        if constexpr (SPLIT) mfma_split1(fa[i], b, acc[j][i], rest[j][i]);
+        else mfma_split1(fa[i], b, acc[j][i]);
+    };
 
 #pragma unroll
     for (int u = 0; u < PA; u++) load_a(u);
@@ -135,7 +142,6 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
     lds_sync();
     auto rows_a = [&](int buf, int i) { return frag(lds + buf * BUF, (BM / 4) * wm + 16 * i, APL); };
     auto rows_b = [&](int buf, int j) { return frag(lds + buf * BUF + 3 * APL, 64 * wn + 16 * j, BPL); };
-    Frag3 fa[I], fb[2];
 #pragma unroll
     for (int i = 0; i < I; i++) fa[i] = rows_a(0, i);
     fb[0] = rows_b(0, 0);
@@ -147,7 +153,9 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
             fb[(j + 1) & 1] = rows_b(cur, j + 1);
             if (j == 0) {                // (fragment by fragment: the last ones are still arriving)
 #pragma unroll
-                for (int i = 0; i < I; i++) mfma_split1(fa[i], fb[0], acc[0][i]);
+                for (int i = 0; i < I; i++) prod(i, 0, fb[0]);
+            } else if constexpr (SPLIT) {
+                mfma_split<I>(fa, fb[j & 1], acc[j], rest[j]);
             } else {
                 mfma_split<I>(fa, fb[j & 1], acc[j]);
             }
@@ -167,11 +175,17 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
         fb[0] = rows_b(nxt, 0);
 #pragma unroll
         for (int i = 0; i < I; i++) {
-            mfma_split1(fa[i], fb[1], acc[J - 1][i]);
+            prod(i, J - 1, fb[1]);
             fa[i] = rows_a(nxt, i);
         }
     }
 
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int j = 0; j < J; j++)
+#pragma unroll
+            for (int i = 0; i < I; i++) acc[j][i] += rest[j][i];
+    }
     // A sum that is not finite comes from operands or products that are not, where a difference of
     // parts is NaN: such values are summed again as they are (through LDS, to index them).
     bool bad = false;

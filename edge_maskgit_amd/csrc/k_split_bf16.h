@@ -68,6 +68,29 @@ __device__ __forceinline__ void mfma_split1(const Frag3& a, const Frag3& b, f32x
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.m, acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.h, acc, 0, 0, 0);
 }
+// both with the five small products in accumulators of their own: the large ones are rounded
+// once per 32 k
+template <int I>
+__device__ __forceinline__ void mfma_split(const Frag3 (&a)[I], const Frag3& b, f32x4 (&acc)[I], f32x4 (&rest)[I]) {
+    auto go = [&](bf16x8 Frag3::*pa, const bf16x8& vb, f32x4(&s)[I]) {
+#pragma unroll
+        for (int i = 0; i < I; i++) s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i].*pa, vb, s[i], 0, 0, 0);
+    };
+    go(&Frag3::h, b.h, acc);
+    go(&Frag3::l, b.h, rest);
+    go(&Frag3::h, b.l, rest);
+    go(&Frag3::m, b.m, rest);
+    go(&Frag3::m, b.h, rest);
+    go(&Frag3::h, b.m, rest);
+}
+__device__ __forceinline__ void mfma_split1(const Frag3& a, const Frag3& b, f32x4& acc, f32x4& rest) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.h, acc, 0, 0, 0);
+    rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.l, b.h, rest, 0, 0, 0);
+    rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.l, rest, 0, 0, 0);
+    rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.m, rest, 0, 0, 0);
+    rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.m, b.h, rest, 0, 0, 0);
+    rest = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.h, b.m, rest, 0, 0, 0);
+}
 
 // LDS hand-over inside a K step: this wave's LDS accesses are done, then the workgroup barrier; the
 // global loads in flight (into registers) stay in flight, which __syncthreads() would wait for

@@ -605,21 +605,23 @@ hipError_t launch_conv2d_f32(const ConvArgs& a, hipStream_t s) {
 bool conv_pk_narrow(int OC) { return OC <= NBN; }
 
 ConvPkPlan conv_pk_plan(int M, int OC, int K) {
-    // Split K when one image's output tiles give fewer than 384 workgroups: up to about 512
-    // workgroups, each split keeping >= 9 16-wide slabs. Measured on the decoder's convs at
-    // one image (split targets 128..1024 workgroups): shorter splits lose to their partial
-    // planes (16 x 16 x 512 -> 512: 31.5 us at 9 slabs per split, 39.1 at 5; the 8-slab 1x1
-    // conv at 128 x 128: 16.7 us unsplit, 30.6 in 4 splits), while the 64-128 px levels want
-    // about 512 workgroups. The plan does not depend on the batch, so an image's sums are the
-    // same whatever it is batched with.
+    // Split K when one image's output tiles are fewer than 192, up to about 256 workgroups, each split
+    // keeping >= 18 16-wide slabs (nine 32-deep steps of k_conv2d_split). Measured on the decoder's
+    // convs, one / two images, against the 512 workgroups of >= 9 slabs that two smaller workgroups per
+    // CU wanted: 64 x 64 x 256 37.7 / 61.3 us against 40.2 / 77.3, 128 x 128 x 128 40.5 / 65.6 against
+    // 42.9 / 81.6, 16 x 16 x 512 26.3 / 26.4 against 25.3 / 31.7 (fewer partial planes to write and
+    // add). The 16-channel tiles keep 512 workgroups of >= 9 slabs. The plan does not depend on the
+    // batch, so an image's sums are the same whatever it is batched with.
     ConvPkPlan p{1, K};
-    const int bm = conv_pk_narrow(OC) ? NBM : PBM, bn = conv_pk_narrow(OC) ? NBN : PBN;
+    const bool nar = conv_pk_narrow(OC);
+    const int bm = nar ? NBM : PBM, bn = nar ? NBN : PBN;
+    const int target = nar ? 512 : 256, least = nar ? 9 : 18;
     const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((OC + bn - 1) / bn);
     const int slabs = K / PBK;
-    const int want = (int)std::min<int64_t>((512 + tiles - 1) / tiles, slabs / 9);
-    if (tiles >= 384 || want < 2) return p;
+    const int want = (int)std::min<int64_t>((target + tiles - 1) / tiles, slabs / least);
+    if (tiles >= target * 3 / 4 || want < 2) return p;
     int per = (slabs + want - 1) / want;
-    if (K % 32 == 0 && !conv_pk_narrow(OC)) per = (per + 1) & ~1;   // whole 32-deep steps (launch_conv_split)
+    if (K % 32 == 0 && !nar) per = (per + 1) & ~1;   // whole 32-deep steps (launch_conv_split)
     p.kps = per * PBK;
     p.splits = (slabs + per - 1) / per;
     return p;
