@@ -225,6 +225,88 @@ __global__ __launch_bounds__(256, 2) void k_conv2d_pkn(ConvPkArgs a) {
                    M, acc[i]);
 }
 
+// conv_out (OC <= 4, 3 x 3, stride 1, pad 1, rows of 4k pixels): on MFMA tiles of 16 channels 13 of 16
+// columns are padding and every input value is gathered nine times. Here a lane computes 4
+// neighbouring pixels of every channel from the 3 x 6 inputs of one input channel (three 16-byte
+// and six 4-byte buffer loads, taps outside the image past the range), the weights broadcast from
+// LDS; the 8 waves of a workgroup take IC / 8 input channels each for the same 256 pixels, and their
+// partial sums are added in wave order. 108 FMAs per channel and lane bound it (256 x 256 x 128 -> 3:
+// 6.3 us of VALU; measured 48 -> 18 us per image).
+template <int OCN>
+__global__ __launch_bounds__(512) void k_conv2d_out(ConvPkArgs a) {
+    constexpr int WP = OCN * 9 + (4 - OCN * 9 % 4) % 4;      // floats per input channel, whole 16 bytes
+    extern __shared__ __attribute__((aligned(16))) float sm[];   // weights [IC][WP], then partials [8][4 OCN][64]
+    const int M = a.OW * a.OH, IC = a.IC, OC = a.OC;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (int i = tid; i < IC * OCN * 9; i += 512) {
+        const int ic = i % IC, ot = i / IC;                  // ot = oc * 9 + tap
+        sm[ic * WP + ot] = ot / 9 < OC ? a.wpk[(size_t)ot * IC + ic] : 0.f;
+    }
+    __syncthreads();
+    const int n = blockIdx.y, p = 4 * (blockIdx.x * 64 + lane);
+    const int ow = p % a.OW, oh = p / a.OW;
+    const uint32_t plane = (uint32_t)(a.IW * a.IH) * 4;
+    const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.in + (size_t)n * IC * a.IW * a.IH), (short)0, (int)((uint32_t)IC * plane), 0x00020000);
+    const uint32_t NO = 0x80000000u;
+    uint32_t vm[3], vl[3], vr[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const int ih = oh - 1 + r;
+        const bool in = p < M && (uint32_t)ih < (uint32_t)a.IH;
+        const uint32_t o = (uint32_t)(ih * a.IW + ow) * 4;
+        vm[r] = in ? o : NO;
+        vl[r] = in && ow > 0 ? o - 4 : NO;
+        vr[r] = in && ow + 4 < a.IW ? o + 16 : NO;
+    }
+    float acc[OCN][4];
+#pragma unroll
+    for (int o = 0; o < OCN; o++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[o][e] = 0.f;
+    const int per = IC / 8, c0 = wave * per;
+#pragma unroll 2
+    for (int c = c0; c < c0 + per; c++) {
+        const uint32_t so = (uint32_t)c * plane;
+        float x[3][6];
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            const f32x4 m = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rin, (int)vm[r], (int)so, 0));
+            x[r][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rin, (int)vl[r], (int)so, 0));
+            x[r][5] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rin, (int)vr[r], (int)so, 0));
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[r][1 + e] = m[e];
+        }
+        float w[WP];
+#pragma unroll
+        for (int q = 0; q < WP / 4; q++) *(f32x4*)&w[4 * q] = *(const f32x4*)&sm[c * WP + 4 * q];
+#pragma unroll
+        for (int t = 0; t < 9; t++)
+#pragma unroll
+            for (int o = 0; o < OCN; o++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[o][e] = fmaf(w[9 * o + t], x[t / 3][t % 3 + e], acc[o][e]);
+    }
+    float* red = sm + IC * WP;
+#pragma unroll
+    for (int o = 0; o < OCN; o++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) red[(wave * 4 * OCN + 4 * o + e) * 64 + lane] = acc[o][e];
+    __syncthreads();
+    for (int i = tid; i < OC * 256; i += 512) {
+        const int oc = i >> 8, px = i & 255, pp = blockIdx.x * 256 + px;
+        if (pp >= M) continue;
+        const float* q = red + (4 * oc + (px & 3)) * 64 + (px >> 2);
+        float v = q[0];
+#pragma unroll
+        for (int s = 1; s < 8; s++) v += q[s * 4 * OCN * 64];
+        const size_t idx = ((size_t)n * OC + oc) * M + pp;
+        if (a.bias) v = v + a.bias[oc];
+        if (a.resid) v = v + a.resid[idx];
+        a.out[idx] = v;
+    }
+}
+
 // out[i] = ((sum over splits in order of part[s][i]) + bias[oc]) + resid[i]
 __global__ __launch_bounds__(256) void k_conv_reduce(const float* __restrict__ part, int splits, int64_t total,
                                                      int M, int OC, const float* __restrict__ bias,
@@ -602,6 +684,13 @@ hipError_t launch_conv2d_f32(const ConvArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// k_conv2d_out's shapes (a workgroup per 256 pixels: small images keep the 16-channel tiles, 20 x 20 x
+// 256 15 against 30 us) within 31-bit offsets
+static bool conv_out_ok(const ConvPkArgs& a) {
+    return a.OC <= 4 && a.KW == 3 && a.KH == 3 && a.stride == 1 && a.pad == 1 && a.OW % 4 == 0 && a.IC % 8 == 0 &&
+           a.IC <= 128 && a.OW * a.OH >= 4096 && (int64_t)a.IC * a.IW * a.IH * 4 < (1ll << 31);
+}
+
 bool conv_pk_narrow(int OC) { return OC <= NBN; }
 
 ConvPkPlan conv_pk_plan(int M, int OC, int K) {
@@ -646,6 +735,14 @@ hipError_t launch_conv_pack(const float* ker, float* wpk, int IC, int taps, int 
 hipError_t launch_conv2d_pk(const ConvPkArgs& a0, float* ws, hipStream_t s) {
     const int M = a0.OW * a0.OH, K = a0.IC * a0.KW * a0.KH;
     if (M == 0 || a0.OC == 0 || a0.N == 0) return hipSuccess;
+    if (conv_out_ok(a0)) {
+        const dim3 grid((unsigned)((M + 255) / 256), (unsigned)a0.N);
+        const unsigned ocn = a0.OC <= 3 ? 3 : 4, wp = (ocn * 9 + 3) / 4 * 4;
+        const unsigned lds = (unsigned)(a0.IC * wp + 8 * 4 * ocn * 64) * 4;      // <= 51 KB
+        if (ocn == 3) hipLaunchKernelGGL(k_conv2d_out<3>, grid, dim3(512), lds, s, a0);
+        else hipLaunchKernelGGL(k_conv2d_out<4>, grid, dim3(512), lds, s, a0);
+        return hipGetLastError();
+    }
     const ConvPkPlan p = conv_pk_plan(M, a0.OC, K);
     ConvPkArgs a = a0;
     a.splits = p.splits;

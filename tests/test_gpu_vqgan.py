@@ -35,12 +35,12 @@ def ctx():
 
 # kernels: IC % 16 == 0 packed tap-major MFMA ("pk": OC > 16, with IC % 32 == 0 on three bf16 parts
 # per value, else on fp32 MFMA; "pkn": 256 x 16 for OC <= 16; split over K when one image's output
-# gives too few workgroups); else OC <= 8 one thread per pixel ("few"), or the reference-layout
+# gives too few workgroups; "out": OC <= 4, 3 x 3 on rows of 4k pixels); else OC <= 8 one thread per pixel ("few"), or the reference-layout
 # MFMA ("gen")
 CONV = [  # IW, IH, IC, N, KW, KH, OC, stride, pad
     (9, 7, 5, 2, 3, 3, 7, 1, 1), (10, 10, 3, 1, 3, 3, 8, 2, 1), (5, 5, 2, 1, 5, 5, 3, 1, 2),
     (7, 7, 4, 1, 3, 3, 3, 1, 0), (32, 32, 128, 1, 3, 3, 3, 1, 1),                     # few, pkn
-    (256, 256, 128, 1, 3, 3, 3, 1, 1), (20, 9, 32, 2, 3, 3, 16, 2, 1),                # pkn
+    (256, 256, 128, 1, 3, 3, 3, 1, 1), (20, 9, 32, 2, 3, 3, 16, 2, 1),                # out, pkn
     (8, 8, 33, 2, 1, 1, 65, 1, 0), (65, 33, 20, 1, 3, 3, 130, 1, 1),                  # gen
     (16, 16, 256, 1, 3, 3, 512, 1, 1), (16, 16, 512, 2, 3, 3, 512, 1, 1),             # pk, split
     (32, 32, 128, 2, 3, 3, 64, 1, 1), (64, 64, 64, 1, 1, 1, 32, 1, 0),                # pk
@@ -48,6 +48,7 @@ CONV = [  # IW, IH, IC, N, KW, KH, OC, stride, pad
     (128, 128, 128, 1, 3, 3, 128, 1, 1), (32, 32, 256, 1, 1, 1, 256, 1, 0),           # pk
     (11, 6, 16, 1, 5, 5, 24, 1, 2),                                                   # pk, 5x5
     (256, 192, 16, 1, 3, 3, 16, 1, 1),                                                # pk, no split
+    (68, 61, 64, 2, 3, 3, 4, 1, 1), (64, 64, 128, 1, 3, 3, 1, 1, 1), (100, 41, 16, 3, 3, 3, 2, 1, 1),  # out
     (16, 15, 32, 1, 1, 1, 17, 1, 0), (17, 15, 64, 3, 3, 3, 129, 1, 1),      # pk: one step; tile edges
     (67, 61, 96, 1, 3, 3, 127, 1, 1), (33, 65, 160, 4, 5, 3, 40, 2, 2),     # 3 and 5 steps per tap
     (257, 200, 32, 1, 3, 3, 64, 1, 1), (240, 221, 64, 1, 1, 1, 128, 1, 0),  # 256-pixel tiles, ragged
@@ -102,6 +103,7 @@ def test_conv2d_batch_invariant(ctx, IW, IH, IC, KW, KH, OC):
 @pytest.mark.parametrize("IW,IH,IC,N,KW,KH,OC,stride,pad", [
     (16, 16, 256, 1, 3, 3, 512, 1, 1), (32, 32, 128, 2, 3, 3, 64, 1, 1), (9, 7, 32, 1, 3, 3, 130, 2, 1),
     (32, 32, 128, 1, 3, 3, 3, 1, 1), (65, 33, 20, 1, 3, 3, 130, 1, 1), (64, 64, 128, 1, 1, 1, 128, 1, 0),
+    (68, 62, 64, 2, 3, 3, 3, 1, 1),
     (256, 192, 16, 1, 3, 3, 16, 1, 1)])
 def test_conv2d_ex_bias_residual_packed(ctx, IW, IH, IC, N, KW, KH, OC, stride, pad):
     """the fused Add nodes: out = (conv + bias) + resid, each rounded as its own node, equal bit for
