@@ -634,7 +634,7 @@ def measure_vqgan(path, steps=5, cpu=True, int8=True):
     if conv_ms:
         a = conv_flop / (conv_ms * 1e-3) / 1e12
         res["roofline_conv_b1"] = {"bound": "mfma", "achieved": round(a, 2), "peak": 157.3, "unit": "TFLOP/s",
-                                   "frac": round(a / 157.3, 4), "kernel": "k_conv2d_pk (+ _pkn, split reduce)",
+                                   "frac": round(a / 157.3, 4), "kernel": "k_conv2d_split (+ k_conv2d_out, split reduce)",
                                    "note": "fp32 MFMA (the reference's conv arithmetic is fp32); all Conv2D "
                                            "nodes of one decode, device time per node"}
     if cpu:

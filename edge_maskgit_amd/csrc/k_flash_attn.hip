@@ -9,8 +9,10 @@
 // The output strides are a parameter too, so the head merge that follows in the reference
 // graph (permute + cont, mg-transformer.cpp:84-85) is written directly.
 //
-// gfx950 mapping (one workgroup = 4 waves = 64 queries of one (b, h); keys in chunks of 64
-// staged once per workgroup in LDS as fp16):
+// Three kernels: k_attn_head (S <= 272: a head's K and V resident in LDS), k_attn_long (longer
+// sequences; both need unit feature strides and aligned rows) and k_flash_attn_f16kv (any strides).
+// gfx950 mapping of the last (one workgroup = 4 waves = 64 queries of one (b, h); keys in chunks of
+// 64 staged once per workgroup in LDS as fp16):
 //  * Scores as S^T = K . Q^T on v_mfma_f32_16x16x32_f16 (two 16-wide d chunks per
 //    instruction, an odd last chunk paired with zeros): fp16 products are exact in fp32, so
 //    only the summation order differs from the reference. The S^T accumulator layout (lane

@@ -183,7 +183,8 @@ int mgh_flash_attn_f16in(mgh_ctx* ctx, const void* d_q16, const void* d_k16, con
 /* ---- fp32 GEMM with the fused epilogue (tied MLM head, F32 FC weights): replaces
  *      k_mul_mat_t and its dispatch (mg-opencl.cpp:60-94, 1429-1440).
  *      y[M][N] = act(x . w^T + bias) + resid; w [N][K], x [M][K]; K % 32 == 0, 16-byte
- *      aligned w and x. ---- */
+ *      aligned w and x. Products of the full 24-bit significands (three bf16 parts per value on
+ *      the bf16 matrix unit), fp32 sums. ---- */
 int mgh_gemm_f32(mgh_ctx* ctx, const float* d_w, int N, int K, const float* d_x, int M,
                  const float* d_bias, int act, const float* d_resid, float* d_y);
 
@@ -225,9 +226,10 @@ int mgh_gemm_f32_batched(mgh_ctx* ctx, const float* d_w, const int64_t w_ne[4], 
  *      mgh_conv2d: the Conv2D node (CPU mg-cpu.cpp:165-190; GPU k_conv2d_t,
  *      mg-opencl.cpp:985-1025, 1535-1566): ker {KW, KH, IC, OC}, out {OW, OH, OC, N} with
  *      OW = (IW + 2 pad - KW) / stride + 1; fp32 products and accumulation; d_out 16-byte aligned.
- *      Kernels: IC % 16 == 0 an fp32-MFMA implicit GEMM over tap-major packed weights (packed
- *      into the context scratch per call, or once by mgh_conv2d_pack_weights; 128 x 128 tiles,
- *      256 x 16 for OC <= 16), with K split across workgroups when one image's output alone
+ *      Kernels: IC % 16 == 0 an implicit GEMM over tap-major packed weights (packed into the
+ *      context scratch per call, or once by mgh_conv2d_pack_weights; IC % 32 == 0 on the bf16
+ *      matrix unit with three parts per fp32 value, else fp32 MFMA; 16-channel tiles for OC <= 16;
+ *      OC <= 4, 3 x 3 on the VALU), with K split across workgroups when one image's output alone
  *      gives too few (per image: results do not depend on the batch); otherwise, for OC <= 8,
  *      one thread per pixel in the reference loop's order (the CPU executor's float operations
  *      exactly), else a 64 x 64 fp32-MFMA implicit GEMM over the reference layout.
