@@ -1,5 +1,5 @@
 // k_vqgan.hip — the VQGAN decoder's ops on gfx950: 2-D convolution as an implicit GEMM on
-// fp32 MFMA, GroupNorm (+ per-channel affine + SiLU), nearest-neighbour upscale.
+// fp32 MFMA (the wide form: k_conv_split.hip), GroupNorm (+ per-channel affine + SiLU), nearest-neighbour upscale.
 //
 // Semantics (layout ne = {W, H, C, N}, W innermost, every tensor contiguous):
 //  * Conv2D: out[n][oc][oh][ow] = sum over (ic, kh, kw) of ker[oc][ic][kh][kw] *
