@@ -160,11 +160,12 @@ __global__ __launch_bounds__(256, DB ? 2 : 4) void k_gemm_f32(GemmF32Args g) {
             const int r = tid / BN + (256 / BN) * q, m = row(r);
             if (m >= M || n >= N) continue;
             const float v = T[r * TP + c];
-            bad = bad || !(fabsf(v) < INFINITY);
-            put(m, v);
+            if (fabsf(v) < INFINITY) put(m, v);
+            else bad = true;
         }
         // A sum that is not finite comes from operands or products that are not, where a
-        // difference of parts is NaN: such values are summed again as they are.
+        // difference of parts is NaN: such values are summed again as they are (and stored once:
+        // resid may be y itself).
         if (bad) {
 #pragma unroll 1
             for (int q = 0; q < HR * BN / 256; q++) {

@@ -388,6 +388,43 @@ def test_gemm_f32_not_finite(ctx, M):
     assert np.abs(y[ok] / np.maximum(np.abs(ref[ok]), 1.0) - ref[ok] / np.maximum(np.abs(ref[ok]), 1.0)).max() <= 2e-5
 
 
+@pytest.mark.parametrize("M", [70, 1100])
+@pytest.mark.parametrize("act", [0, 2])
+def test_gemm_f32_not_finite_epilogue(ctx, M, act):
+    """sums that are redone get bias, activation and residual once, also where the residual is y
+    itself (read and written once per element): equal bit for bit to a residual of its own"""
+    N, K = 1000, 64
+    print(f"gemm_f32 not finite, epilogue M={M} act={act}", flush=True)
+    rng = np.random.default_rng(M + act)
+    w, x = (rng.standard_normal(s).astype(np.float32) for s in ((N, K), (M, K)))
+    bias, resid = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    big = np.finfo(np.float32).max                # its first bf16 part is an infinity
+    x[3, 5], x[M - 1, 0] = np.inf, np.nan
+    x[7] = 0
+    x[7, 2] = big
+    w[:, 2] *= 0.25
+    w[11, 2] = 1.0
+    dW, dX, dB, dR = ctx.upload(w), ctx.upload(x), ctx.upload(bias), ctx.upload(resid)
+    dY = ctx.alloc(M * N * 4)
+    ctx.gemm_f32(dW, N, K, dX, M, dB, act, dR, dY)
+    ctx.gemm_f32(dW, N, K, dX, M, dB, act, dR, dR)
+    y, inplace = ctx.download(dY, (M, N), np.float32), ctx.download(dR, (M, N), np.float32)
+    for t in (dW, dX, dB, dR, dY):
+        ctx.free(t)
+    assert np.array_equal(y.view(np.uint32), inplace.view(np.uint32))
+    with np.errstate(invalid="ignore", over="ignore"):
+        s = np.stack([(x[m].astype(np.float64) * w.astype(np.float64)).sum(-1) for m in range(M)]) + bias
+        s = s.astype(np.float32).astype(np.float64)
+        ref = ((s if act == 0 else s / (1 + np.exp(-s))) + resid).astype(np.float32)
+    assert np.array_equal(np.isnan(y), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(y[inf], ref[inf])
+    ok = np.isfinite(ref)
+    assert ok[7].sum() > N // 2                   # finite sums of the largest value among them
+    # as test_gemm_f32_not_finite: a few fp32 roundings of sums of K terms
+    assert (np.abs(y[ok].astype(np.float64) - ref[ok]) / np.maximum(np.abs(ref[ok]).astype(np.float64), 1.0)).max() <= 2e-5
+
+
 # ---- glue ------------------------------------------------------------------------------
 def test_get_rows_add_copy(ctx):
     print("glue ops", flush=True)
