@@ -85,37 +85,38 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Grow-on-demand activation scratch (like the reference's qx_buf/dx_buf,
-// mg-opencl.cpp:1125-1134). Not allowed while a graph is being captured. The replaced
-// buffer is retired, not freed (stream order keeps it valid for queued work and graphs).
-int ensure_scratch(mgh_ctx* c, size_t need) {
-    if (c->scratch_bytes >= need) return MGH_OK;
+// Grow-on-demand context buffers (like the reference's qx_buf/dx_buf, mg-opencl.cpp:1125-1134).
+// Not allowed while a graph is being captured. The replaced buffer is retired, not freed (stream
+// order keeps it valid for queued work and graphs), and only once the larger one is there: a
+// failed allocation leaves the context as it was. At least doubled, so that retired buffers
+// together stay below the current one; the exact size where twice the old one cannot be had.
+int grow(mgh_ctx* c, void*& buf, size_t& bytes, size_t need, const char* name) {
+    if (bytes >= need) return MGH_OK;
     if (c->capturing)
-        return fail(c, MGH_ERR_ARG, "activation scratch must grow, which is not allowed during "
+        return fail(c, MGH_ERR_ARG, std::string(name) + " must grow, which is not allowed during "
                                     "graph capture (run the call once before capturing)");
-    need = std::max(need, 2 * c->scratch_bytes);
-    if (c->scratch) c->retired.push_back(c->scratch);
-    c->scratch = nullptr;
-    c->scratch_bytes = 0;
-    MGH_HIP(c, hipMalloc(&c->scratch, need), "hipMalloc(scratch)");
-    c->scratch_bytes = need;
+    size_t size = std::max(need, 2 * bytes);
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, size);
+    if (e != hipSuccess && size > need) {
+        (void)hipGetLastError();
+        size = need;
+        e = hipMalloc(&p, size);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return hip_fail(c, e, (std::string("hipMalloc(") + name + ")").c_str());
+    }
+    if (buf) c->retired.push_back(buf);
+    buf = p;
+    bytes = size;
     return MGH_OK;
 }
 
+int ensure_scratch(mgh_ctx* c, size_t need) { return grow(c, c->scratch, c->scratch_bytes, need, "activation scratch"); }
+
 // Split-K workspace of the packed GEMM (partial tiles).
-int ensure_qp_ws(mgh_ctx* c, size_t need) {
-    if (c->qp_ws_bytes >= need) return MGH_OK;
-    if (c->capturing)
-        return fail(c, MGH_ERR_ARG, "split-K workspace must grow, which is not allowed during graph "
-                                    "capture (run the call once before capturing)");
-    need = std::max(need, 2 * c->qp_ws_bytes);
-    if (c->qp_ws) c->retired.push_back(c->qp_ws);
-    c->qp_ws = nullptr;
-    c->qp_ws_bytes = 0;
-    MGH_HIP(c, hipMalloc(&c->qp_ws, need), "hipMalloc(qp_ws)");
-    c->qp_ws_bytes = need;
-    return MGH_OK;
-}
+int ensure_qp_ws(mgh_ctx* c, size_t need) { return grow(c, c->qp_ws, c->qp_ws_bytes, need, "split-K workspace"); }
 
 // The packed GEMM with its split-K plan (workspace from the context).
 int run_gemm_qp(mgh_ctx* c, int wtype, mgh::GemmArgs a, bool dbg) {
@@ -954,8 +955,7 @@ void expand_weights(mgh_ctx* c, mgh::GemmH16Args& a, size_t off) {
     const size_t need = off + (size_t)a.N * a.K * 2;
     if (c->scratch_bytes < need && (c->capturing || (size_t)a.N * a.K * 2 > ((size_t)1 << 28))) return;
     if (ensure_scratch(c, need) != MGH_OK) {
-        c->err.clear();
-        (void)hipGetLastError();
+        c->err.clear();                  // (the scratch there was is still there)
         return;
     }
     char* w16 = (char*)c->scratch + off;
