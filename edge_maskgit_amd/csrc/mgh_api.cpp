@@ -132,13 +132,14 @@ int run_gemm_qp(mgh_ctx* c, int wtype, mgh::GemmArgs a, bool dbg) {
     return MGH_OK;
 }
 
-// The fp16 dequantize-fused GEMM with its split-K plan (workspace from the context).
-int run_gemm_h16(mgh_ctx* c, mgh::GemmH16Args a) {
+// The fp16 dequantize-fused GEMM with its split-K plan (workspace from the context): the plan of
+// weight form plan_wq.
+int run_gemm_h16(mgh_ctx* c, mgh::GemmH16Args a, int plan_wq) {
     if (mgh::use_gemv_h16(a.M, a.K)) {
         MGH_HIP(c, mgh::launch_gemv_h16(a, c->stream), "k_gemv_fc");
         return MGH_OK;
     }
-    const mgh::H16Plan p = mgh::gemm_h16_plan(a.M, a.N, a.K, a.xf != nullptr, a.wq);
+    const mgh::H16Plan p = mgh::gemm_h16_plan(a.M, a.N, a.K, a.xf != nullptr, plan_wq);
     a.splits = p.splits;
     if (p.splits > 1) {
         if (int r = ensure_qp_ws(c, p.ws_bytes)) return r;
@@ -949,19 +950,22 @@ bool expand_pays(int M, int N) { return M >= (N <= 1024 ? 700 : 1024); }
 
 // Weights of a call on Q4_K bytes with many rows: expanded to fp16 in the context scratch (from `off`
 // on) and multiplied in that form. A call that cannot have the scratch (not while a graph is
-// captured, or the allocation fails) decodes in the K loop as before.
-void expand_weights(mgh_ctx* c, mgh::GemmH16Args& a, size_t off) {
-    if (a.wq != MGH_WTYPE_Q4_K || !expand_pays(a.M, a.N)) return;
+// captured, or the allocation fails) decodes the same values in the K loop, under the same plan, so
+// that its sums are the same whatever scratch it found. Returns the weight form whose plans the call
+// takes.
+int expand_weights(mgh_ctx* c, mgh::GemmH16Args& a, size_t off) {
+    if (a.wq != MGH_WTYPE_Q4_K || !expand_pays(a.M, a.N)) return a.wq;
     const size_t need = off + (size_t)a.N * a.K * 2;
-    if (c->scratch_bytes < need && (c->capturing || (size_t)a.N * a.K * 2 > ((size_t)1 << 28))) return;
+    if (c->scratch_bytes < need && (c->capturing || (size_t)a.N * a.K * 2 > ((size_t)1 << 28))) return 0;
     if (ensure_scratch(c, need) != MGH_OK) {
         c->err.clear();                  // (the scratch there was is still there)
-        return;
+        return 0;
     }
     char* w16 = (char*)c->scratch + off;
-    if (mgh::launch_expand_q4(a.w, w16, a.N, a.K, c->stream) != hipSuccess) return;
+    if (mgh::launch_expand_q4(a.w, w16, a.N, a.K, c->stream) != hipSuccess) return 0;
     a.w = w16;
     a.wq = 0;
+    return 0;
 }
 
 // The dequantize-fused FC entry points, for either weight form: wq 0 (fp16 [N][K] from
@@ -976,8 +980,8 @@ int gemm_h16_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, int K
     a.x = (const _Float16*)x16; a.w = w; a.wq = wq;
     a.bias = bias; a.resid = resid; a.y = y16 ? nullptr : y; a.y16 = y16;
     a.M = M; a.N = N; a.K = K; a.act = act;
-    expand_weights(c, a, 0);
-    return run_gemm_h16(c, a);
+    const int plan_wq = expand_weights(c, a, 0);
+    return run_gemm_h16(c, a, plan_wq);
 }
 
 int gemm_h16_ln_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, int K, const void* x16, int M,
@@ -1004,8 +1008,8 @@ int gemm_h16_ln_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, in
     a.bias = bias; a.resid = resid; a.y = y;
     a.M = M; a.N = N; a.K = K; a.act = act;
     const size_t y_b = no_y ? round256((size_t)M * N * 4) : 0;
-    expand_weights(c, a, y_b);
-    const mgh::H16Plan p = mgh::gemm_h16_plan(M, N, K, false, a.wq);
+    const int plan_wq = expand_weights(c, a, y_b);
+    const mgh::H16Plan p = mgh::gemm_h16_plan(M, N, K, false, plan_wq);
     if (!mgh::use_gemv_h16(M, K) && p.splits > 1 && act == 0) {
         // the split-K reduce normalizes each row as it leaves: one launch fewer
         if (int r = ensure_qp_ws(c, p.ws_bytes)) return r;
@@ -1020,7 +1024,7 @@ int gemm_h16_ln_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, in
         if (int r = ensure_scratch(c, y_b)) return r;
         a.y = y = (float*)c->scratch;
     }
-    if (int r = run_gemm_h16(c, a)) return r;
+    if (int r = run_gemm_h16(c, a, plan_wq)) return r;
     MGH_HIP(c, mgh::launch_layernorm_affine(y, gamma, beta, y_ln, M, N, eps, emit, codes, dx, s4, c->stream),
             "k_layernorm_affine");
     return MGH_OK;
@@ -1048,7 +1052,7 @@ int gemm_h16_f32in_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N,
     a.M = M; a.N = N; a.K = K; a.act = act;
     const bool pass = round_act_pass(M, N);
     const size_t x_b = pass ? round256((size_t)M * K * 2) : 0;
-    expand_weights(c, a, x_b);
+    const int plan_wq = expand_weights(c, a, x_b);
     if (!pass) {
         a.xf = x;                               // rounded while the GEMM reads them
     } else {
@@ -1058,7 +1062,7 @@ int gemm_h16_f32in_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N,
         MGH_HIP(c, mgh::launch_f32_to_f16(x, (_Float16*)c->scratch, (int64_t)M * K, c->stream), "k_f32_to_f16");
         a.x = (const _Float16*)c->scratch;
     }
-    return run_gemm_h16(c, a);
+    return run_gemm_h16(c, a, plan_wq);
 }
 
 int check_dq(mgh_ctx* c, const char* fn, int wtype, int N, int K) {

@@ -82,3 +82,32 @@ assert "k_expand_q4" in kernels()
 c.close()
 assert fake.fake_used() == 0
 """)
+
+
+def test_q4k_plan_does_not_depend_on_scratch():
+    """a Q4_K call captured without scratch takes the tile plan of the expanded call (and is accepted
+    wherever its own plan was: no split-K workspace that only the other plan would need)"""
+    run("""
+def fc():
+    out = []
+    for k, n, g in launches():
+        if k.startswith("k_gemm_fc") or k == "k_gemv_fc":
+            out.append((k, re.findall(r"L[a-z]+([0-9]+)E", n)[:-1], g))      # all but the weight form
+    return out
+
+for M in (700, 1023, 1024, 1025, 2056, 4097):
+    for N, K in ((100, 256), (768, 768), (1024, 1024), (2304, 768), (3072, 768), (4096, 512)):
+        for f, x in ((c.gemm_dq_f32in, X), (c.gemm_dq, X)):
+            if f == c.gemm_dq_f32in and M * N >= 4096 * 3072:
+                continue                       # the rounding pass needs scratch of its own
+            fresh = ema.Context(0)
+            g = getattr(fresh, f.__name__)
+            fresh.graph_begin()
+            g(12, W, N, K, x, M, B, 1, R, Y)
+            fresh.graph_end().destroy()
+            captured = fc()
+            g(12, W, N, K, x, M, B, 1, R, Y)
+            eager = fc()
+            fresh.close()
+            assert captured and captured == eager, (M, N, K, captured, eager)
+""")

@@ -426,3 +426,36 @@ def test_q4k_expanded_ln_and_capture():
         c.gemm_h16_ln(dP, N, K, dX, M, None, 0, dR, None, dG, dE, 1e-12, ln)
         c.gemm_dq_ln(q, dQ, N, K, dX, M, None, 0, dR, None, dG, dE, 1e-12, ln2)
         assert np.array_equal(c.download(ln, (M, N), np.float32), c.download(ln2, (M, N), np.float32))
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 768, 768), (1025, 2304, 768), (1030, 3072, 256), (1025, 768, 3072), (4100, 772, 512)])
+def test_q4k_sums_do_not_depend_on_scratch(M, N, K):
+    """a call captured on a context without scratch decodes in the K loop, the eager call expands
+    the weights: the same values under the same plan, so equal bit for bit (split-K plans get their
+    workspace from a Q8_0 call of the same plan first)"""
+    print(f"q4k captured / eager M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    q = ema.WTYPE_Q4_K
+    wq = oracle.quantize(q, (rng.standard_normal((N, K)) * 0.02).astype(np.float32))
+    x, resid = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    with ema.Context(0) as c, ema.Context(0) as e:
+        dW, dX, dX16, dR = c.upload(wq), c.upload(x), c.upload(x.astype(np.float16)), c.upload(resid)
+        dQ, dP = c.alloc(ema.packed_weight_bytes_dq(q, N, K)), c.alloc(ema.packed_weight_bytes_f16(N, K))
+        c.pack_weights_dq(q, dW, N, K, dQ)
+        c.pack_weights_f16(q, dW, N, K, dP)
+        y = [c.alloc(M * N * 4) for _ in range(2)]
+        for call, x_, warm in ((lambda k, *a: k.gemm_dq_f32in(q, *a), dX, c.gemm_h16_f32in),
+                               (lambda k, *a: k.gemm_dq(q, *a), dX16, c.gemm_h16)):
+            warm(dP, N, K, x_, M, None, 1, dR, y[0])     # the fp16 form: no scratch (M * N is below the rounding pass)
+            c.graph_begin()
+            call(c, dQ, N, K, x_, M, None, 1, dR, y[0])
+            g = c.graph_end()
+            call(e, dQ, N, K, x_, M, None, 1, dR, y[1])
+            want = e.download(y[1], (M, N), np.float32)
+            assert np.isfinite(want).all() and want.any()
+            for _ in range(3):
+                c.fill_u32(y[0], 0, M * N)
+                g.launch()
+                c.sync()
+                assert np.array_equal(c.download(y[0], (M, N), np.float32).view(np.uint32), want.view(np.uint32))
+            g.destroy()
