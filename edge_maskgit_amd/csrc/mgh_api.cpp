@@ -939,22 +939,33 @@ int mgh_f32_to_f16(mgh_ctx* c, const float* x, int64_t n, void* x16) {
 namespace {
 
 // Decoding Q4_K in the K loop costs ~23 VALU per fragment in every activation tile; expanding the
-// weights to fp16 first costs a launch and their fp16 bytes (4-5 us) and lets the call run the
-// fp16 form's plans. Measured per FC, cold buffers, fp32 / fp16 activations, K loop against expanded:
-// M = 4097 QKV 46.0 / 32.5 against 39.2 / 30.2 us, out 22.2 / 20.5 against 16.3 / 13.9, up 52.5 / 44.0
-// against 48.1 / 41.8, down 72.8 / 51.5 against 45.3 / 38.0; M = 1025 QKV 19.2 / 15.6 against 17.7 /
-// 16.8, up 24.3 / 22.1 against 21.8 / 18.9; M = 700 QKV 15.3 / 13.0 against 17.4 / 14.1 but out 16.0 /
-// 9.9 against 10.5 / 9.1, down 25.6 / 24.1 against 23.9 / 21.7. Q8_0 decodes in 1.5 VALU per weight:
-// its K loop stays ahead.
-bool expand_pays(int M, int N) { return M >= (N <= 1024 ? 700 : 1024); }
+// weights to fp16 first costs a launch and their fp16 bytes (5-7 us) and lets the call run the
+// fp16 form's plans. Measured per FC (M = 700 .. 4112, N = 768 .. 4096, K = 768 .. 3072, six
+// buffers in turn), K loop / expanded in us:
+//  * N <= 1024: expanded wins from 700 rows on (out-proj 16.5 / 10.9, fp16 rows 9.9 / 9.1; down-proj
+//    25.4 / 23.8, 23.8 / 21.4; at M = 4112 22.2 / 15.7 and 72.9 / 50.3);
+//  * wider, fp16 rows: the K loop holds while its 64-row tiles run in about one round, to ~200 128 x
+//    128 tiles (M = 1285 QKV 15.7 / 17.3, M = 1024 up-proj 15.9 / 17.2, N = 1536 12.4 / 13.0; beyond:
+//    M = 1025 up-proj 20.6 / 17.7, M = 1542 QKV 20.4 / 16.8);
+//  * wider, fp32 rows: to ~140 (M = 1285, N = 1536 14.6 / 15.5; M = 1025 QKV 18.4 / 17.6, M = 1542, N =
+//    1536 18.5 / 16.2), but past N = 3072 to 2048 rows: there the fp16 weights leave two workgroups
+//    per CU where the bytes leave three (M = 1285, N = 4096 28.4 / 32.5; M = 2056 41.4 / 36.0);
+//  * wider, under 1024 rows: the K loop (M = 700 QKV 15.3 / 17.4, fp16 rows 13.0 / 14.1).
+// Q8_0 decodes in 1.5 VALU per weight: its K loop stays ahead.
+bool expand_pays(int M, int N, bool xf32) {
+    if (N <= 1024) return M >= 700;
+    if (M < 1024) return false;
+    const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    return xf32 ? t128 >= 140 && (N <= 3072 || M >= 2048) : t128 >= 200;
+}
 
 // Weights of a call on Q4_K bytes with many rows: expanded to fp16 in the context scratch (from `off`
 // on) and multiplied in that form. A call that cannot have the scratch (not while a graph is
 // captured, or the allocation fails) decodes the same values in the K loop, under the same plan, so
 // that its sums are the same whatever scratch it found. Returns the weight form whose plans the call
 // takes.
-int expand_weights(mgh_ctx* c, mgh::GemmH16Args& a, size_t off) {
-    if (a.wq != MGH_WTYPE_Q4_K || !expand_pays(a.M, a.N)) return a.wq;
+int expand_weights(mgh_ctx* c, mgh::GemmH16Args& a, bool xf32, size_t off) {
+    if (a.wq != MGH_WTYPE_Q4_K || !expand_pays(a.M, a.N, xf32)) return a.wq;
     const size_t need = off + (size_t)a.N * a.K * 2;
     if (c->scratch_bytes < need && (c->capturing || (size_t)a.N * a.K * 2 > ((size_t)1 << 28))) return 0;
     if (ensure_scratch(c, need) != MGH_OK) {
@@ -980,7 +991,7 @@ int gemm_h16_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, int K
     a.x = (const _Float16*)x16; a.w = w; a.wq = wq;
     a.bias = bias; a.resid = resid; a.y = y16 ? nullptr : y; a.y16 = y16;
     a.M = M; a.N = N; a.K = K; a.act = act;
-    const int plan_wq = expand_weights(c, a, 0);
+    const int plan_wq = expand_weights(c, a, false, 0);
     return run_gemm_h16(c, a, plan_wq);
 }
 
@@ -1008,7 +1019,7 @@ int gemm_h16_ln_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N, in
     a.bias = bias; a.resid = resid; a.y = y;
     a.M = M; a.N = N; a.K = K; a.act = act;
     const size_t y_b = no_y ? round256((size_t)M * N * 4) : 0;
-    const int plan_wq = expand_weights(c, a, y_b);
+    const int plan_wq = expand_weights(c, a, false, y_b);
     const mgh::H16Plan p = mgh::gemm_h16_plan(M, N, K, false, plan_wq);
     if (!mgh::use_gemv_h16(M, K) && p.splits > 1 && act == 0) {
         // the split-K reduce normalizes each row as it leaves: one launch fewer
@@ -1052,7 +1063,7 @@ int gemm_h16_f32in_any(mgh_ctx* c, const char* fn, int wq, const void* w, int N,
     a.M = M; a.N = N; a.K = K; a.act = act;
     const bool pass = round_act_pass(M, N);
     const size_t x_b = pass ? round256((size_t)M * K * 2) : 0;
-    const int plan_wq = expand_weights(c, a, x_b);
+    const int plan_wq = expand_weights(c, a, true, x_b);
     if (!pass) {
         a.xf = x;                               // rounded while the GEMM reads them
     } else {

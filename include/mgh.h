@@ -332,7 +332,13 @@ int mgh_gemm_h16_y16(mgh_ctx* ctx, const void* d_wp16, int N, int K, const void*
  *      weight; rows padded to a multiple of 16; buffer size mgh_packed_weight_bytes_dq). The
  *      kernels decode each weight to d*q, resp. (d*sc)*q - dmin*m rounded once to fp16 -- the
  *      value mgh_pack_weights_f16 stores -- as the MFMA fragments are read, so results equal
- *      mgh_gemm_h16's for the same tile plan. Shapes and alignment as mgh_gemm_h16 (K % 64 == 0,
+ *      mgh_gemm_h16's for the same tile plan. Q4_K calls with many rows (from 700 for N <= 1024; for
+ *      wider outputs from 1024 rows and about 140 tiles of 128 x 128 outputs with fp32 rows, 200 with
+ *      fp16 rows) take mgh_gemm_h16's plan, and so its bits: they decode the weights once per call into
+ *      the context scratch (2 N K bytes, grown on demand up to 256 MiB and kept), or, where the
+ *      scratch cannot be had (it would have to grow while a graph is captured; no memory), in the
+ *      K loop under that plan: the same values, slower. A call that ran once before a capture
+ *      expands in the graph too. Shapes and alignment as mgh_gemm_h16 (K % 64 == 0,
  *      Q4_K K % 256 == 0, N % 4 == 0, N <= 2097152, 16-byte aligned operands). ---- */
 size_t mgh_packed_weight_bytes_dq(int wtype, int N, int K);
 /* raw Q8_0 / Q4_K blocks (GGUF layout, any byte alignment) -> fp32 [N][K], the values the

@@ -111,3 +111,21 @@ for M in (700, 1023, 1024, 1025, 2056, 4097):
             fresh.close()
             assert captured and captured == eager, (M, N, K, captured, eager)
 """)
+
+
+def test_q4k_expands_where_it_measured_faster():
+    """both sides of the rule's lines, fp32 and fp16 rows (times beside the rule)"""
+    run("""
+rule = [  # M, N, expanded with fp32 rows, with fp16 rows
+    (699, 768, 0, 0), (700, 768, 1, 1), (700, 1024, 1, 1), (4112, 768, 1, 1), (4097, 1536, 1, 1),
+    (1285, 1536, 0, 0), (1542, 1536, 1, 0), (2056, 1536, 1, 1), (1023, 2304, 0, 0), (1023, 4096, 0, 0), (1025, 2304, 1, 0), (1285, 2304, 1, 0),
+    (1542, 2304, 1, 1), (1024, 3072, 1, 0), (1025, 3072, 1, 1), (1285, 4096, 0, 1), (1542, 4096, 0, 1),
+    (2056, 4096, 1, 1)]
+for M, N, f32, f16 in rule:
+    c.gemm_dq_f32in(12, W, N, 768, X, M, B, 0, None, Y)
+    assert ("k_expand_q4" in kernels()) == bool(f32), (M, N, "fp32 rows")
+    c.gemm_dq_y16(12, W, N, 768, X, M, B, 0, None, Y)
+    assert ("k_expand_q4" in kernels()) == bool(f16), (M, N, "fp16 rows")
+    c.gemm_dq_f32in(8, W, N, 768, X, M, B, 0, None, Y)
+    assert "k_expand_q4" not in kernels()
+""")
