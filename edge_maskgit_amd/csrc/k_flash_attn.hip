@@ -593,8 +593,9 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
     // staging: this key group's chunk c, K pieces (key, 4 features) and V blocks (4 keys x 4
     // features; lanes run over 4 feature blocks, then key blocks: 64-byte row segments). Buffer
     // loads over the head's rows: loop-invariant lane offsets, the chunk in the scalar offset,
-    // rows past S outside the range (zeros), so the loop spends no vector instruction on
-    // addresses or bounds.
+    // rows past S outside the range (zeros; the check takes lane and scalar offset together, also
+    // where the scalar one alone is past the range: measured), so the loop spends no vector
+    // instruction on addresses or bounds.
     constexpr int EB = I16 ? 2 : 4;      // bytes per element
     typedef std::conditional_t<I16, f16x4, f32x4> E4;
     const uint32_t ext = (uint32_t)(((int64_t)(S - 1) * a.st[1] + D) * EB);
@@ -800,7 +801,7 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
         store(0);
         for (int it = 0; it + 1 < nit; it++) {
             __syncthreads();             // this buffer is filled, the other one no longer read
-            load((it + 1) * KS + kg);
+            if (KS == 1 || (it + 1) * KS + kg < nch) load((it + 1) * KS + kg);   // (else: the last chunk again, never read)
             if (active) step(std::false_type{}, it & 1, it * KS + kg);
             store((it + 1) & 1);
         }

@@ -223,6 +223,70 @@ def test_flash_attn_long(ctx, D, S, H, B, pad, opad):
     assert np.array_equal(o16.view(np.uint16), o.astype(np.float16).view(np.uint16))
 
 
+# S % 64 = 1, 17, 33, 0 keys in the last chunk, an odd and an even number of chunks for the two key
+# groups, and the 128-query form (50 heads); heads interleaved in rows and image after image, so that
+# the row after an image's last is the next image's first.
+@pytest.mark.parametrize("D,S,H", [(48, 577, 2), (48, 593, 2), (32, 353, 2), (64, 640, 2), (16, 273, 3), (48, 417, 50),
+                                   (64, 385, 50)])
+def test_flash_attn_long_reads_no_row_past_the_image(ctx, D, S, H):
+    """an image's output is the same bits whether the next image's q/k/v are numbers or NaN"""
+    print(f"flash_attn_long past the image D={D} S={S} H={H}", flush=True)
+    rng = np.random.default_rng(D + S)
+    E = H * D
+    x = rng.standard_normal((2, S, 3 * E)).astype(np.float32)
+    do = ctx.alloc(2 * S * E * 4)
+    outs = []
+    for fill in (None, np.nan, np.inf):
+        if fill is not None:
+            x[1] = fill
+        d = ctx.upload(x)
+        ctx.flash_attn_f16kv(d.ptr, d.ptr + 4 * E, d.ptr + 8 * E, (1, 3 * E, D, 3 * E * S), D, S, H, 2, D ** -0.5, do,
+                             o_strides=(1, E, D, E * S))
+        outs.append(ctx.download(do, (2, S, E), np.float32))
+        ctx.free(d)
+    ctx.free(do)
+    assert np.isfinite(outs[0]).all()
+    for o in outs[1:]:
+        assert np.array_equal(o[0].view(np.uint32), outs[0][0].view(np.uint32))
+        assert np.isnan(o[1]).all()
+
+
+@pytest.mark.parametrize("D,S,H", [(48, 577, 2), (48, 417, 50), (32, 353, 2), (64, 640, 2)])
+def test_flash_attn_long_not_finite(ctx, D, S, H):
+    """NaN and infinities (also fp32 values past fp16's largest) in q, k and v of one head: a score of
+    -inf is a weight of zero, one of +inf or NaN makes the query's row NaN, a value that is not
+    finite spoils its feature; everything else is what the finite softmax gives"""
+    print(f"flash_attn_long not finite D={D} S={S} H={H}", flush=True)
+    rng = np.random.default_rng(S)
+    E = H * D
+    x = rng.standard_normal((S, 3, H, D)).astype(np.float32)
+    x[5, 0, 0, 3] = np.nan                        # a query
+    x[7, 0, 0, 2] = np.inf
+    x[100, 1, 0, 1] = -np.inf                     # a key: scores of either infinity, by the query's sign
+    x[S - 1, 1, 1, 0] = 7e4                       # fp16: inf, in the last chunk
+    x[70, 2, 0, 4], x[S - 2, 2, 0, 6] = np.nan, np.inf
+    d, do = ctx.upload(x), ctx.alloc(S * E * 4)
+    ctx.flash_attn_f16kv(d.ptr, d.ptr + 4 * E, d.ptr + 8 * E, (1, 3 * E, D, 3 * E * S), D, S, H, 1, D ** -0.5, do,
+                         o_strides=(1, E, D, E * S))
+    o = ctx.download(do, (S, H, D), np.float32)
+    for t in (d, do):
+        ctx.free(t)
+    with np.errstate(invalid="ignore", over="ignore"):
+        h = x.astype(np.float16).astype(np.float64)
+        for i in range(min(H, 3)):
+            sc = (h[:, 0, i, None, :] * h[None, :, 1, i, :]).sum(-1) * D ** -0.5
+            p = np.exp(sc - sc.max(-1, keepdims=True))
+            p /= p.sum(-1, keepdims=True)
+            bad = ~np.isfinite(h[:, 2, i]).all(0)                     # features with a value that is not finite
+            ref = p @ np.where(np.isfinite(h[:, 2, i]), h[:, 2, i], 0.0)
+            rows = np.isfinite(p).all(-1)
+            assert i or (0 < rows.sum() < S and bad.sum() == 2)
+            assert np.isnan(o[~rows, i]).all()
+            assert not np.isfinite(o[:, i][:, bad]).any()
+            got, want = o[rows, i][:, ~bad], ref[rows][:, ~bad]
+            assert np.isfinite(got).all() and np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
 def test_flash_attn_long_strides(ctx):
     """The same attention through strides the long kernel does not take (features two elements
     apart: the kernel for any strides) and through ones it takes: both within 2e-5 max|ref| of
