@@ -557,38 +557,41 @@ constexpr int LVLD = LKT + 8;            // V^T row stride (halves): 9 16-byte s
 template <int DC>
 constexpr int kLongKLD = DC <= 2 ? 40 : 72;   // K row stride (halves): 32 or 64 features + 8
 
-template <int DC, int QG, int QT, int KS, bool I16>
-__global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull, int heads) {
+// queries [body, S) are a split block's: at most `tail` of them, past a multiple of `gran`
+struct LongCut {
+    int gran, tail;
+};
+template <int QG, int QT, int KS, int SEQ>
+constexpr LongCut kLongCut = KS * SEQ == 1 ? LongCut{16 * QT * QG, 16 * QT} : LongCut{64, 16};
+
+template <int DC, int QG, int QT, int KS, int SEQ, bool I16>
+__global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nblk, int body, int heads) {
     constexpr int D = 16 * DC, KLD = kLongKLD<DC>, KC = (DC + 1) / 2, NW = QG * KS;
+    constexpr int G = KS * SEQ;          // key groups
+    constexpr int NV = G == 1 ? NW : 8;  // parts a split block's keys are taken in
+    static_assert((KS == 1 || SEQ == 1) && NV % NW == 0, "");
     constexpr int GT = 64 * QG;          // threads per key group
     constexpr int KV4 = LKT * D / 4;     // 16-byte pieces of a chunk's K
     constexpr int UK = (KV4 + GT - 1) / GT, VB = LKT / 4 * (D / 4), UV = (VB + GT - 1) / GT;
     constexpr int CH = LKT * KLD + D * LVLD;     // halves per chunk buffer
     constexpr int MR = QT * (4 * DC + 2);   // floats a lane hands over in the merge
-    constexpr int STAGE = 2 * KS * CH * 2, MERGE = NW * 64 * MR * 4;
-    __shared__ __attribute__((aligned(16))) char lds[STAGE > MERGE ? STAGE : MERGE];
+    constexpr int STAGE = 2 * KS * CH * 2, MERGE = NV * 64 * MR * 4, STASH = SEQ > 1 ? NW * 64 * MR * 4 : 0;
+    __shared__ __attribute__((aligned(16))) char lds[STAGE + STASH > MERGE ? STAGE + STASH : MERGE];
 
     const int S = a.S;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = wave / QG, qg = wave - kg * QG, gt = tid - kg * GT;
     const int l16 = lane & 15, lg = lane >> 4;
-    // whole blocks first, each XCD taking contiguous runs of (head, block) so that its L2 holds
-    // few heads' K and V; then the heads' partial blocks
-    const int nf = nfull * heads;
-    int hb, qb;
-    if ((int)blockIdx.x < nf) {
-        const int lid = xcd_remap(blockIdx.x, nf);
-        hb = lid / nfull, qb = lid - hb * nfull;
-    } else {
-        hb = blockIdx.x - nf, qb = nfull;
-    }
+    // each XCD takes contiguous runs of (head, block), so that its L2 holds few heads' K and V; then
+    // the heads' split blocks
+    const int nf = nblk * heads;
+    const bool split = (int)blockIdx.x >= nf;
+    const int lid = split ? (int)blockIdx.x - nf : xcd_remap(blockIdx.x, nf);
+    const int hb = split ? lid : lid / nblk, qb = lid - hb * nblk;
     const int h = hb % a.H, b = hb / a.H;
     const int64_t base = (int64_t)b * a.st[3] + (int64_t)h * a.st[2];
-    const int q0b = qb * 16 * QT * QG;
-    // a partial block with one wave's queries: its waves split the keys
-    const bool split = NW > 1 && S - q0b <= 16 * QT;
-    const int q0 = q0b + (split ? 0 : 16 * QT * qg);
-    const bool active = q0 < S;
+    const int q0 = split ? body : (qb * QG + qg) * 16 * QT;
+    const bool active = q0 < (split ? S : body);
 
     // staging: this key group's chunk c, K pieces (key, 4 features) and V blocks (4 keys x 4
     // features; lanes run over 4 feature blocks, then key blocks: 64-byte row segments). Buffer
@@ -665,8 +668,9 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
             if (d < D) qf[qt][c] = load_h8<I16, false>(a.q, a.q16, qrow + d);
         }
     }
-    // the features between D and the padded width meet zeros of Q: they only have to be finite
-    if (D % 32) {
+    // the features between D and the padded width meet zeros of Q: they only have to be finite (a split
+    // block keeps its parts' states there instead)
+    if (D % 32 && !split) {
         for (int i = tid; i < 2 * KS * LKT; i += 64 * NW)
 #pragma unroll
             for (int e = 0; e < 2; e++)
@@ -680,13 +684,46 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
     // query l16) and the row sums (every register of S1)
     float mref[QT], S1[QT];
     f32x4 O[QT][DC];
+    auto reset = [&] {
 #pragma unroll
-    for (int qt = 0; qt < QT; qt++) {
-        mref[qt] = -1e30f;
-        S1[qt] = 0.f;
+        for (int qt = 0; qt < QT; qt++) {
+            mref[qt] = -1e30f;
+            S1[qt] = 0.f;
 #pragma unroll
-        for (int c = 0; c < DC; c++) O[qt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+            for (int c = 0; c < DC; c++) O[qt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    reset();
+    // this state in LDS ([MR][64 lanes] per part), and two parts' merged: the earlier part's is this
+    // one (LATER: the one in LDS)
+    constexpr int MQ = 4 * DC + 2;
+    auto put = [&](float* w) {
+        w += lane;
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++) {
+            w[qt * MQ * 64] = mref[qt];
+            w[(qt * MQ + 1) * 64] = S1[qt];
+#pragma unroll
+            for (int c = 0; c < DC; c++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) w[(qt * MQ + 2 + 4 * c + r) * 64] = O[qt][c][r];
+        }
+    };
+    auto merge = [&](const float* w, auto later) {
+        w += lane;
+#pragma unroll
+        for (int qt = 0; qt < QT; qt++) {
+            const float mo = w[qt * MQ * 64], mn = fmaxf(mref[qt], mo);
+            const float al = __builtin_amdgcn_exp2f(mref[qt] - mn), be = __builtin_amdgcn_exp2f(mo - mn);
+            auto add = [&](float x, float y) { return decltype(later)::value ? fmaf(x, al, y * be) : fmaf(y, be, x * al); };
+            mref[qt] = mn;
+            S1[qt] = add(S1[qt], w[(qt * MQ + 1) * 64]);
+#pragma unroll
+            for (int c = 0; c < DC; c++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) O[qt][c][r] = add(O[qt][c][r], w[(qt * MQ + 2 + 4 * c + r) * 64]);
+        }
+    };
 
     // NT key tiles from key0 on: kfrag(t, i) is the K fragment of tile t, features 32 i + 8 lg + j;
     // vfrag(p, c) the V^T fragment of tiles 2p, 2p + 1, feature 16 c + l16. (MASK is a property
@@ -718,7 +755,7 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
                         for (int qt = 0; qt < QT; qt++) sc[qt][t][r] = -INFINITY;
         }
         float mx[QT];
-        bool up = false;
+        bool up[QT], any = false;        // (per query tile: a tile's sums do not depend on the wave's other one)
 #pragma unroll
         for (int qt = 0; qt < QT; qt++) {
             float v = -INFINITY;
@@ -728,12 +765,13 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
                 v = fmaxf(fmaxf(v, sc[qt][t][2]), sc[qt][t][3]);
             }
             mx[qt] = v * scale2;
-            up = up || mx[qt] > mref[qt] + 15.f;
+            up[qt] = __any(mx[qt] > mref[qt] + 15.f);
+            any = any || up[qt];
         }
-        if (__any(up)) {
+        if (any) {
 #pragma unroll
             for (int qt = 0; qt < QT; qt++) {
-                float v = fmaxf(mx[qt] - 7.f, mref[qt]);
+                float v = up[qt] ? fmaxf(mx[qt] - 7.f, mref[qt]) : mref[qt];
                 v = fmaxf(v, __shfl_xor(v, 16));
                 v = fmaxf(v, __shfl_xor(v, 32));
                 const float al = __builtin_amdgcn_exp2f(mref[qt] - v);
@@ -799,17 +837,44 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
         };
         load(kg);
         store(0);
-        for (int it = 0; it + 1 < nit; it++) {
-            __syncthreads();             // this buffer is filled, the other one no longer read
-            if (KS == 1 || (it + 1) * KS + kg < nch) load((it + 1) * KS + kg);   // (else: the last chunk again, never read)
-            if (active) step(std::false_type{}, it & 1, it * KS + kg);
-            store((it + 1) & 1);
+        if constexpr (SEQ == 1) {
+            for (int it = 0; it + 1 < nit; it++) {
+                __syncthreads();         // this buffer is filled, the other one no longer read
+                if (KS == 1 || (it + 1) * KS + kg < nch) load((it + 1) * KS + kg);   // (else: the last chunk again, never read)
+                if (active) step(std::false_type{}, it & 1, it * KS + kg);
+                store((it + 1) & 1);
+            }
+            __syncthreads();
+            const int c = (nit - 1) * KS + kg;
+            if (active && c < nch) step(std::true_type{}, (nit - 1) & 1, c);
+        } else {
+            // the key groups one after the other, the first one's state kept in LDS meanwhile
+            float* stash = (float*)(lds + STAGE) + wave * MR * 64;
+            int buf = 0;
+#pragma unroll 1
+            for (int g = 0; g < SEQ; g++) {
+                int c = g;
+                for (; c + SEQ < nch; c += SEQ) {
+                    __syncthreads();
+                    load(c + SEQ);
+                    if (active) step(std::false_type{}, buf, c);
+                    buf ^= 1;
+                    store(buf);
+                }
+                __syncthreads();
+                if (g + 1 < SEQ) load(g + 1);
+                if (active) step(std::true_type{}, buf, c);
+                if (g + 1 < SEQ) {
+                    buf ^= 1;
+                    store(buf);
+                    put(stash);
+                    reset();
+                }
+            }
+            merge(stash, std::true_type{});
         }
-        __syncthreads();
-        const int c = (nit - 1) * KS + kg;
-        if (active && c < nch) step(std::true_type{}, (nit - 1) & 1, c);
     } else {
-        // 32-key groups wave, wave + NW, ..., each wave's fragments straight from memory (rows
+        // part v takes 32-key groups v, v + NV, ..., each wave's fragments straight from memory (rows
         // past S and features past D outside the buffer range: zeros). Holding the next group's
         // values as well would cost the registers that let this block share a CU with two whole
         // ones
@@ -838,60 +903,43 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
                         vr[cc][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsv, o, (int)so, 0));
                 }
         };
-        for (int g = wave; g < ng; g += NW) {
-            fetch(g);
-            f16x8 kf[2][KC], vf[DC];
+#pragma unroll 1
+        for (int v = wave; v < NV; v += NW) {
+            for (int g = v; g < ng; g += NV) {
+                fetch(g);
+                f16x8 kf[2][KC], vf[DC];
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+                for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int i = 0; i < KC; i++)
+                    for (int i = 0; i < KC; i++)
 #pragma unroll
-                    for (int j = 0; j < 8; j++) kf[t][i][j] = (_Float16)kr[t][i][j >> 2][j & 3];
+                        for (int j = 0; j < 8; j++) kf[t][i][j] = (_Float16)kr[t][i][j >> 2][j & 3];
 #pragma unroll
-            for (int cc = 0; cc < DC; cc++)
+                for (int cc = 0; cc < DC; cc++)
 #pragma unroll
-                for (int j = 0; j < 8; j++) vf[cc][j] = (_Float16)vr[cc][j];
-            compute(std::integral_constant<int, 2>{}, std::true_type{}, 32 * g, [&](int t, int i) { return kf[t][i]; },
-                    [&](int, int cc) { return vf[cc]; });
+                    for (int j = 0; j < 8; j++) vf[cc][j] = (_Float16)vr[cc][j];
+                compute(std::integral_constant<int, 2>{}, std::true_type{}, 32 * g, [&](int t, int i) { return kf[t][i]; },
+                        [&](int, int cc) { return vf[cc]; });
+            }
+            if (NV > NW) {
+                put((float*)lds + v * MR * 64);
+                reset();
+            }
         }
     }
 
-    // merge: the waves that share queries (the key groups; with split, all waves) hand their
-    // (reference, sum, O) to the first of them
+    // merge, in the order of the parts: the waves that share queries (the key groups; in a split block
+    // all of them) hand their state to the first of them
     if (KS > 1 || split) {
         __syncthreads();
-        float* mg = (float*)lds;         // [wave][MR][64 lanes]
+        float* mg = (float*)lds;         // [part][MR][64 lanes]
         const bool first = kg == 0 && (!split || qg == 0);
-        if (!first && active) {
-            float* w = mg + wave * MR * 64 + lane;
-#pragma unroll
-            for (int qt = 0; qt < QT; qt++) {
-                w[(qt * (4 * DC + 2)) * 64] = mref[qt];
-                w[(qt * (4 * DC + 2) + 1) * 64] = S1[qt];
-#pragma unroll
-                for (int c = 0; c < DC; c++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) w[(qt * (4 * DC + 2) + 2 + 4 * c + r) * 64] = O[qt][c][r];
-            }
-        }
+        if (!first && active && !(split && NV > NW)) put(mg + wave * MR * 64);
         __syncthreads();
         if (!first) return;
+        // (NV > NW: part 0 merged into the empty state is itself: its scale is exp2(0), the other's exp2(-inf))
         const int step = split ? 1 : QG;
-        for (int o = wave + step; o < NW; o += step) {
-            const float* w = mg + o * MR * 64 + lane;
-#pragma unroll
-            for (int qt = 0; qt < QT; qt++) {
-                const float mo = w[(qt * (4 * DC + 2)) * 64], mn = fmaxf(mref[qt], mo);
-                const float al = __builtin_amdgcn_exp2f(mref[qt] - mn), be = __builtin_amdgcn_exp2f(mo - mn);
-                mref[qt] = mn;
-                S1[qt] = fmaf(w[(qt * (4 * DC + 2) + 1) * 64], be, S1[qt] * al);
-#pragma unroll
-                for (int c = 0; c < DC; c++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        O[qt][c][r] = fmaf(w[(qt * (4 * DC + 2) + 2 + 4 * c + r) * 64], be, O[qt][c][r] * al);
-            }
-        }
+        for (int o = split && NV > NW ? 0 : wave + step; o < (split ? NV : NW); o += step) merge(mg + o * MR * 64, std::false_type{});
     }
     if (!active) return;
     const bool vec = a.os[0] == 1 && ((a.os[1] | a.os[2] | a.os[3]) & 3) == 0 &&
@@ -925,26 +973,42 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nfull,
     }
 }
 
-template <int DC, int QG, int QT, int KS>
+template <int DC, int QG, int QT, int KS, int SEQ>
 void launch_long_t(const FaArgs& a, hipStream_t s) {
-    const int qb = 16 * QT * QG, nfull = a.S / qb, heads = a.H * a.B;
-    const dim3 grid((unsigned)(heads * (nfull + (a.S % qb ? 1 : 0)))), block(64 * QG * KS);
-    if (a.q16) hipLaunchKernelGGL((k_attn_long<DC, QG, QT, KS, true>), grid, block, 0, s, a, nfull, heads);
-    else hipLaunchKernelGGL((k_attn_long<DC, QG, QT, KS, false>), grid, block, 0, s, a, nfull, heads);
+    constexpr LongCut cut = kLongCut<QG, QT, KS, SEQ>;
+    const int r = a.S % cut.gran, body = r && r <= cut.tail ? a.S - r : a.S;
+    const int qb = 16 * QT * QG, nblk = (body + qb - 1) / qb, heads = a.H * a.B;
+    const dim3 grid((unsigned)(heads * (nblk + (body < a.S ? 1 : 0)))), block(64 * QG * KS);
+    if (a.q16) hipLaunchKernelGGL((k_attn_long<DC, QG, QT, KS, SEQ, true>), grid, block, 0, s, a, nblk, body, heads);
+    else hipLaunchKernelGGL((k_attn_long<DC, QG, QT, KS, SEQ, false>), grid, block, 0, s, a, nblk, body, heads);
 }
 
-// Few query blocks (one image of up to ~1500 tokens): 64 queries and two key groups per workgroup,
-// so that every CU has a workgroup of eight waves; from about 200 128-query blocks (120 at D = 64,
-// whose 64-query form holds 150 registers) 128 queries per workgroup, each K / V fragment serving
-// two query tiles. Measured, 16 heads, D = 48, fp32 q/k/v, (64 queries x 2 key groups) against 128
-// queries: S = 600 10.0 / 15.4 us, 1025 18.0 / 23.3, 2049 48.9 / 45.3, 4097 156 / 124, S = 1025
-// with 4 images 45.7 / 37.9; D = 64: S = 1500, 12 heads 36.9 / 33.3. One key group with 64
-// queries lies between the two everywhere but within 10% of the better one.
+// From 200 128-query blocks per image (120 at D = 64, whose 64-query form holds 150 registers) 128
+// queries per workgroup, each K / V fragment serving two query tiles, one key group. An image with fewer
+// (up to ~1500 tokens) takes its keys in two groups, so that one image gives every CU a workgroup of
+// eight waves: 64 queries and the groups side by side, or, in a call with many blocks, 128 queries and
+// the groups one after the other, the same sums: an image's result does not depend on its batch.
+// Measured, 16 heads, D = 48, fp32 q/k/v:
+//  * one image, two groups side by side against 128 queries and one group: S = 600 10.0 / 15.4 us, 1025
+//    18.0 / 23.3, 2049 48.9 / 45.3, 4097 156 / 124 (D = 64: S = 1500, 12 heads 36.9 / 33.3);
+//  * a batch, side by side against one after the other: S = 600 x 3 16.7 / 17.6, 801 x 2 18.4 / 20.9, 1025 x
+//    4 46.9 / 44.0, 1025 x 16 186 / 149; D = 64: 513 x 8 44.7 / 33.2. Side by side while its 64-query
+//    blocks run in one round (two per CU; D = 64: one), or while the 128-query blocks' last round is so
+//    empty that they take longer (a CU's round of two waves per SIMD: 1.5 times as long; 1300 x 3: 50 /
+//    62). With one group instead, whose sums are others, a batch took up to 15% less (1025 x 4: 38.8): the
+//    first group's state costs LDS and so one of three workgroups per CU.
 template <int DC>
 hipError_t launch_long(const FaArgs& a, hipStream_t s) {
-    const int64_t nb = (int64_t)a.H * a.B * ((a.S + 127) / 128);
-    if (nb < (DC <= 3 ? 200 : 120)) launch_long_t<DC, 4, 1, 2>(a, s);
-    else launch_long_t<DC, 4, 2, 1>(a, s);
+    constexpr LongCut cut = kLongCut<4, 1, 2, 1>;
+    const int64_t heads = (int64_t)a.H * a.B;
+    const bool tail = a.S % cut.gran && a.S % cut.gran <= cut.tail;
+    const int64_t n64 = heads * ((a.S - (tail ? cut.tail : 0) + 63) / 64), n128 = heads * ((a.S - (tail ? cut.tail : 0) + 127) / 128);
+    if ((int64_t)a.H * ((a.S + 127) / 128) >= (DC <= 3 ? 200 : 120))
+        launch_long_t<DC, 4, 2, 1, 1>(a, s);
+    else if (n64 + (tail ? heads : 0) <= (DC <= 3 ? 512 : 256) || 2 * ((n64 + 255) / 256) < 3 * ((n128 + 255) / 256))
+        launch_long_t<DC, 4, 1, 2, 1>(a, s);
+    else
+        launch_long_t<DC, 4, 2, 1, 2>(a, s);
     return hipGetLastError();
 }
 

@@ -161,7 +161,8 @@ int mgh_layernorm_affine(mgh_ctx* ctx, const float* d_x, const float* d_gamma, c
 /* ---- flash attention with fp16 K/V: replaces k_flash_attention_h and its dispatch
  *      (mg-opencl.cpp:859-937, 1483-1511). q/k/v are {D,S,H,B} views with element strides
  *      strides[4] (d, s, h, b); the output has element strides o_strides[4], or is the
- *      contiguous {D,S,H,B} tensor when o_strides is NULL. D in {16, 32, 48, 64}. ---- */
+ *      contiguous {D,S,H,B} tensor when o_strides is NULL. D in {16, 32, 48, 64}. An image's
+ *      result does not depend on how many images share the call. ---- */
 int mgh_flash_attn_f16kv(mgh_ctx* ctx, const float* d_q, const float* d_k, const float* d_v,
                          const int64_t strides[4], int D, int S, int H, int B, float scale,
                          float* d_o, const int64_t o_strides[4]);

@@ -223,6 +223,44 @@ def test_flash_attn_long(ctx, D, S, H, B, pad, opad):
     assert np.array_equal(o16.view(np.uint16), o.astype(np.float16).view(np.uint16))
 
 
+# one image's call takes two key groups side by side, a batch of them one after the other (from 200
+# 128-query blocks in the call, 120 at D = 64), an image with as many blocks of its own one group
+@pytest.mark.parametrize("D,S,H,B", [(48, 273, 16, 6), (48, 400, 16, 4), (48, 577, 16, 3), (48, 592, 10, 5), (48, 600, 16, 3),
+                                     (32, 385, 16, 4), (16, 321, 16, 5), (64, 513, 16, 3), (64, 450, 16, 2), (64, 528, 8, 4),
+                                     (48, 1025, 8, 4), (48, 1025, 25, 2)])
+def test_flash_attn_long_batch_invariant(ctx, D, S, H, B):
+    """an image's output is the same bits alone and in a batch, for fp32 and fp16 outputs and inputs"""
+    print(f"flash_attn_long batch D={D} S={S} H={H} B={B}", flush=True)
+    rng = np.random.default_rng(D + S + B)
+    E = H * D
+    x = rng.standard_normal((B, S, 3, E)).astype(np.float32)
+    x[:, :, 1] *= np.linspace(0.2, 4.0, S)[None, :, None]       # the softmax reference moves
+    st, ost = (1, 3 * E, D, 3 * E * S), (1, E, D, E * S)
+    d, d16 = ctx.upload(x), ctx.upload(x.astype(np.float16))
+    do, dh, one = ctx.alloc(B * S * E * 4), ctx.alloc(B * S * E * 2), ctx.alloc(S * E * 4)
+
+    def attn(fn, base, elem, n, out, **kw):
+        fn(base, base + elem * E, base + 2 * elem * E, st, D, S, H, n, D ** -0.5, *out, **kw)
+
+    attn(ctx.flash_attn_f16kv, d.ptr, 4, B, (do,), o_strides=ost)
+    attn(ctx.flash_attn_f16kv_o16, d.ptr, 4, B, (dh,), o_strides=ost)
+    o, o16 = ctx.download(do, (B, S, E), np.float32), ctx.download(dh, (B, S, E), np.float16)
+    if S <= 512:
+        attn(ctx.flash_attn_f16in, d16.ptr, 2, B, (do, None, ost))
+        assert np.array_equal(ctx.download(do, (B, S, E), np.float32).view(np.uint32), o.view(np.uint32))
+    assert np.array_equal(o16.view(np.uint16), o.astype(np.float16).view(np.uint16))
+    for b in (0, B - 1):
+        attn(ctx.flash_attn_f16kv, d.ptr + 12 * E * S * b, 4, 1, (one,), o_strides=ost)
+        assert np.array_equal(ctx.download(one, (S, E), np.float32).view(np.uint32), o[b].view(np.uint32))
+    for t in (d, d16, do, dh, one):
+        ctx.free(t)
+    # both forms against float64, on one head
+    h = x[B - 1].astype(np.float16).astype(np.float64).reshape(S, 3, H, D)[:, :, H - 1]
+    sc = h[:, 0] @ h[:, 1].T * D ** -0.5
+    p = np.exp(sc - sc.max(-1, keepdims=True))
+    assert _rel(o[B - 1].reshape(S, H, D)[:, H - 1], p @ h[:, 2] / p.sum(-1, keepdims=True)) <= 2e-5
+
+
 # S % 64 = 1, 17, 33, 0 keys in the last chunk, an odd and an even number of chunks for the two key
 # groups, and the 128-query form (50 heads); heads interleaved in rows and image after image, so that
 # the row after an image's last is the next image's first.
