@@ -35,6 +35,8 @@ namespace mgh {
 namespace {
 
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ f16x8 cat8(f16x4 a, f16x4 b) {
@@ -528,8 +530,9 @@ hipError_t launch_head(const FaArgs& a, hipStream_t s) {
 // and KS key groups of QG waves that take every KS-th chunk; the key groups' (max, sum, O) are
 // merged through LDS at the end. The work is VALU-bound (4.5 operations per score, one of them
 // a quarter-rate exp2), so:
-//  * the products, the P = hi + lo split, the row sums from the matrix unit and the transposed
-//    P . V are k_attn_head's; one 32-deep MFMA covers 32 features / keys, whose order inside a
+//  * the products, the row sums from the matrix unit and the transposed P . V are k_attn_head's,
+//    as is P = hi + lo but for the rounding: both parts to nearest (v_cvt_pk_f16_f32, as fast as the
+//    truncating form), at most 1.2e-7 of P lost against 3.6e-7; one 32-deep MFMA covers 32 features / keys, whose order inside a
 //    fragment is free as long as both operands share it, so K rows (padded with zeros to 32) and
 //    V^T rows (keys permuted within 32: position 8 lg + 4 (t % 2) + r holds key 16 (t % 2) + 4 lg
 //    + r) are read with one conflict-free 16-byte read per fragment;
@@ -550,8 +553,8 @@ hipError_t launch_head(const FaArgs& a, hipStream_t s) {
 // block with a single wave's queries is split over the keys instead, each wave reading its own
 // fragments from memory without the staging or its barriers.
 // Measured (16 heads, D = 48, one image) against the kernel for any strides: S = 1025 114 -> 18 us,
-// S = 4097 549 -> 121 us (16-bit MFMA work at full rate: ~50 us, VALU ~55 us), error against
-// 64 bits 3.8e-7 -> 2.3e-7 and 6.6e-7 -> 2.9e-7.
+// S = 4097 549 -> 122 us (16-bit MFMA work at full rate: ~50 us, VALU ~55 us), error against
+// 64 bits 3.8e-7 -> 2.1e-7 and 6.6e-7 -> 2.8e-7.
 constexpr int LKT = 64;                  // keys per chunk
 constexpr int LVLD = LKT + 8;            // V^T row stride (halves): 9 16-byte slots
 template <int DC>
@@ -801,11 +804,12 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nblk, 
                     e[j] = __builtin_amdgcn_exp2f(fmaf(sc[qt][2 * p + j / 4][j % 4], scale2, -mref[qt]));
                 u32x4 hi, lo;
                 auto u = [](auto v) { return __builtin_bit_cast(uint32_t, v); };
+                auto rne = [](float a, float b) { return __builtin_convertvector(f32x2{a, b}, f16x2); };
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const auto hh = __builtin_amdgcn_cvt_pkrtz(e[2 * j], e[2 * j + 1]);
+                    const f16x2 hh = rne(e[2 * j], e[2 * j + 1]);
                     hi[j] = u(hh);
-                    lo[j] = u(__builtin_amdgcn_cvt_pkrtz(fmaf((float)hh[0], m1, e[2 * j]), fmaf((float)hh[1], m1, e[2 * j + 1])));
+                    lo[j] = u(rne(fmaf((float)hh[0], m1, e[2 * j]), fmaf((float)hh[1], m1, e[2 * j + 1])));
                 }
                 const f16x8 ph = __builtin_bit_cast(f16x8, hi), pl = __builtin_bit_cast(f16x8, lo);
 #pragma unroll

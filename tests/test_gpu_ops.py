@@ -223,6 +223,31 @@ def test_flash_attn_long(ctx, D, S, H, B, pad, opad):
     assert np.array_equal(o16.view(np.uint16), o.astype(np.float16).view(np.uint16))
 
 
+def test_flash_attn_long_weights_are_rounded_to_nearest(ctx):
+    """the softmax weights enter P . V as two fp16 parts rounded to nearest. One key in 32 has a lower
+    score s (another for every query) and value 1, the others value 0, so the output follows the
+    weight of s alone. RMS of its relative error over 8 heads of queries, with exp2, scale and division
+    in fp32: measured 1.43e-7 and 1.15e-7; with truncated parts 1.62e-7 and 1.35e-7"""
+    rms = []
+    for D, S in ((16, 1024), (48, 640)):
+        H, E = 8, 8 * D
+        rng = np.random.default_rng(3)
+        x = np.zeros((S, 3, H, D), np.float32)
+        x[:, 0, :, 0] = -rng.uniform(0.5, 7, (S, H)).astype(np.float16)
+        x[::32, 1:, :, 0] = 1.0
+        d, do = ctx.upload(x), ctx.alloc(S * E * 4)
+        ctx.flash_attn_f16kv(d.ptr, d.ptr + 4 * E, d.ptr + 8 * E, (1, 3 * E, D, 3 * E * S), D, S, H, 1, 1.0, do,
+                             o_strides=(1, E, D, E * S))
+        o = ctx.download(do, (S, H, D), np.float32)[:, :, 0].astype(np.float64)
+        for t in (d, do):
+            ctx.free(t)
+        p = np.exp(x[:, 0, :, 0].astype(np.float64)) * (S // 32)
+        ref = p / (p + S - S // 32)
+        rms.append(float(np.sqrt((((o - ref) / ref) ** 2).mean())))
+    print("  rms", rms)
+    assert rms[0] <= 1.53e-7 and rms[1] <= 1.25e-7
+
+
 # one image's call takes two key groups side by side, a batch of them one after the other (from 200
 # 128-query blocks in the call, 120 at D = 64), an image with as many blocks of its own one group
 @pytest.mark.parametrize("D,S,H,B", [(48, 273, 16, 6), (48, 400, 16, 4), (48, 577, 16, 3), (48, 592, 10, 5), (48, 600, 16, 3),
