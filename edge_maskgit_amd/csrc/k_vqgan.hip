@@ -693,24 +693,28 @@ static bool conv_out_ok(const ConvPkArgs& a) {
 
 bool conv_pk_narrow(int OC) { return OC <= NBN; }
 
-ConvPkPlan conv_pk_plan(int M, int OC, int K) {
-    // Split K when one image's output tiles are fewer than 192, up to about 256 workgroups, each split
-    // keeping >= 18 16-wide slabs (nine 32-deep steps of k_conv2d_split). Measured on the decoder's
-    // convs, one / two images, against the 512 workgroups of >= 9 slabs that two smaller workgroups per
-    // CU wanted: 64 x 64 x 256 37.7 / 61.3 us against 40.2 / 77.3, 128 x 128 x 128 40.5 / 65.6 against
-    // 42.9 / 81.6, 16 x 16 x 512 26.3 / 26.4 against 25.3 / 31.7 (fewer partial planes to write and
-    // add). The 16-channel tiles keep 512 workgroups of >= 9 slabs. The plan does not depend on the
-    // batch, so an image's sums are the same whatever it is batched with.
+ConvPkPlan conv_pk_plan(const ConvPkArgs& a) {
+    // Split K while one image's output tiles are fewer than 3/4 of a target number of workgroups, up to
+    // that target, each split keeping a least number of 16-wide slabs. The plan does not depend on
+    // the batch, so an image's sums are the same whatever it is batched with.
+    //  * k_conv2d_split (one workgroup per CU): 256 workgroups, 18 slabs (nine 32-deep steps). Measured
+    //    on the decoder's convs, one / two images, against 512 of 9 slabs: 64 x 64 x 256 37.7 / 61.3
+    //    us against 40.2 / 77.3, 128 x 128 x 128 40.5 / 65.6 against 42.9 / 81.6, 16 x 16 x 512 26.3 /
+    //    26.4 against 25.3 / 31.7 (fewer partial planes to write and add);
+    //  * k_conv2d_pk and the 16-channel tiles (two or more smaller workgroups per CU): 512 workgroups,
+    //    9 slabs. k_conv2d_pk, one image, against 256 of 18: 64 x 64 x 48 -> 128 22.6 against 41.9 us,
+    //    32 x 32 x 80 -> 128 20.6 / 38.5, 16 x 16 x 240 -> 512 25.1 / 36.7, 64 x 64 x 144 -> 256 44.1 / 46.1.
+    const int M = a.OW * a.OH, OC = a.OC, K = a.IC * a.KW * a.KH;
     ConvPkPlan p{1, K};
-    const bool nar = conv_pk_narrow(OC);
+    const bool nar = conv_pk_narrow(OC), wide = !nar && conv_split_ok(a);
     const int bm = nar ? NBM : PBM, bn = nar ? NBN : PBN;
-    const int target = nar ? 512 : 256, least = nar ? 9 : 18;
+    const int target = wide ? 256 : 512, least = wide ? 18 : 9;
     const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((OC + bn - 1) / bn);
     const int slabs = K / PBK;
     const int want = (int)std::min<int64_t>((target + tiles - 1) / tiles, slabs / least);
     if (tiles >= target * 3 / 4 || want < 2) return p;
     int per = (slabs + want - 1) / want;
-    if (K % 32 == 0 && !nar) per = (per + 1) & ~1;   // whole 32-deep steps (launch_conv_split)
+    if (wide) per = (per + 1) & ~1;      // whole 32-deep steps
     p.kps = per * PBK;
     p.splits = (slabs + per - 1) / per;
     return p;
@@ -719,9 +723,9 @@ ConvPkPlan conv_pk_plan(int M, int OC, int K) {
 // images per split launch: grid z = images x splits stays within 65535
 static int conv_pk_group(int N, int splits) { return std::min(N, 65535 / splits); }
 
-size_t conv_pk_ws_bytes(int M, int OC, int N, int K) {
-    const ConvPkPlan p = conv_pk_plan(M, OC, K);
-    return p.splits > 1 ? (size_t)p.splits * conv_pk_group(N, p.splits) * OC * (size_t)M * sizeof(float) : 0;
+size_t conv_pk_ws_bytes(const ConvPkArgs& a) {
+    const ConvPkPlan p = conv_pk_plan(a);
+    return p.splits > 1 ? (size_t)p.splits * conv_pk_group(a.N, p.splits) * a.OC * (size_t)(a.OW * a.OH) * sizeof(float) : 0;
 }
 
 hipError_t launch_conv_pack(const float* ker, float* wpk, int IC, int taps, int OC, hipStream_t s) {
@@ -733,7 +737,7 @@ hipError_t launch_conv_pack(const float* ker, float* wpk, int IC, int taps, int 
 }
 
 hipError_t launch_conv2d_pk(const ConvPkArgs& a0, float* ws, hipStream_t s) {
-    const int M = a0.OW * a0.OH, K = a0.IC * a0.KW * a0.KH;
+    const int M = a0.OW * a0.OH;
     if (M == 0 || a0.OC == 0 || a0.N == 0) return hipSuccess;
     if (conv_out_ok(a0)) {
         const dim3 grid((unsigned)((M + 255) / 256), (unsigned)a0.N);
@@ -743,7 +747,7 @@ hipError_t launch_conv2d_pk(const ConvPkArgs& a0, float* ws, hipStream_t s) {
         else hipLaunchKernelGGL(k_conv2d_out<4>, grid, dim3(512), lds, s, a0);
         return hipGetLastError();
     }
-    const ConvPkPlan p = conv_pk_plan(M, a0.OC, K);
+    const ConvPkPlan p = conv_pk_plan(a0);
     ConvPkArgs a = a0;
     a.splits = p.splits;
     a.kps = p.kps;
@@ -768,7 +772,7 @@ hipError_t launch_conv2d_pk(const ConvPkArgs& a0, float* ws, hipStream_t s) {
         a.N = g;
         const dim3 grid(gx, gy, (unsigned)(g * p.splits));
         if (nar) hipLaunchKernelGGL(k_conv2d_pkn<true>, grid, block, 0, s, a);
-        else if (conv_split_ok(a) && a.kps % 32 == 0) launch_conv_split(a, s);
+        else if (conv_split_ok(a)) launch_conv_split(a, s);
         else hipLaunchKernelGGL(k_conv2d_pk<true>, grid, block, 0, s, a);
         const int64_t total = (int64_t)g * out_img;
         const int64_t nb = std::min<int64_t>((total + 255) / 256, 8192);

@@ -738,8 +738,8 @@ int mgh_conv2d_ex(mgh_ctx* c, const float* in, int IW, int IH, int IC, int N, co
         MGH_HIP(c, mgh::launch_conv_pack(ker, (float*)c->scratch, IC, KW * KH, OC, c->stream), "k_conv_pack");
         wpk = (const float*)c->scratch;
     }
-    if (int r = ensure_qp_ws(c, mgh::conv_pk_ws_bytes(M, OC, N, K))) return r;
     mgh::ConvPkArgs a{in, wpk, out, bias, resid, IW, IH, IC, (int)OW, (int)OH, OC, KW, KH, stride, pad, N, 1, K};
+    if (int r = ensure_qp_ws(c, mgh::conv_pk_ws_bytes(a))) return r;
     MGH_HIP(c, mgh::launch_conv2d_pk(a, (float*)c->qp_ws, c->stream), "k_conv2d_pk");
     return MGH_OK;
 }

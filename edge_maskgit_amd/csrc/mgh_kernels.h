@@ -245,8 +245,8 @@ bool conv_pk_narrow(int OC);
 // the same on the bf16 matrix unit (k_conv_split.hip; a.splits and a.kps set, kps % 32 == 0)
 bool conv_split_ok(const ConvPkArgs& a);
 void launch_conv_split(const ConvPkArgs& a, hipStream_t s);
-ConvPkPlan conv_pk_plan(int M, int OC, int K);   // per image: independent of the batch
-size_t conv_pk_ws_bytes(int M, int OC, int N, int K);    // split-K partials, 0 without a split
+ConvPkPlan conv_pk_plan(const ConvPkArgs& a);       // per image: independent of the batch
+size_t conv_pk_ws_bytes(const ConvPkArgs& a);       // split-K partials, 0 without a split
 hipError_t launch_conv_pack(const float* ker, float* wpk, int IC, int taps, int OC, hipStream_t s);
 hipError_t launch_conv2d_pk(const ConvPkArgs& a, float* ws, hipStream_t s);
 // int8 conv (the reference's k_conv2d_i8): weights from launch_conv_quant_w — int8 codes in

@@ -129,3 +129,24 @@ for M, N, f32, f16 in rule:
     c.gemm_dq_f32in(8, W, N, 768, X, M, B, 0, None, Y)
     assert "k_expand_q4" not in kernels()
 """)
+
+
+def test_conv_split_k_follows_the_kernel():
+    """256 workgroups of at least 18 slabs of 16 k for the convolutions on three bf16 parts (one
+    workgroup per CU); 512 of at least 9 for the other packed ones, IC % 32 != 0 or 2 GiB images"""
+    run("""
+for side, ic, oc, ksz in ((64, 48, 128, 3), (16, 48, 512, 3), (32, 80, 128, 3), (16, 240, 512, 3), (64, 144, 256, 3), (64, 128, 128, 3),
+                          (64, 256, 256, 3), (16, 512, 512, 3), (32, 96, 40, 3), (32, 128, 3, 3), (8, 16, 24, 5)):
+    c.conv2d_ex(X, side, side, ic, 1, None, W, ksz, ksz, oc, 1, ksz // 2, None, None, Y)
+    (k, _, grid), *reduce = launches()
+    wide = oc > 16 and ic % 32 == 0
+    assert k == ("k_conv2d_split" if wide else "k_conv2d_pkn" if oc <= 16 else "k_conv2d_pk"), k
+    target, least = (256, 18) if wide else (512, 9)
+    bm, bn = (256, 16) if oc <= 16 else (128, 128)
+    tiles, slabs = -(-side * side // bm) * -(-oc // bn), ic * ksz * ksz // 16
+    want = min(-(-target // tiles), slabs // least)
+    per = slabs if tiles >= target * 3 // 4 or want < 2 else -(-slabs // want)
+    per += per % 2 if wide else 0
+    assert grid[2] == -(-slabs // per), (side, ic, oc, grid, per)
+    assert [r[0] for r in reduce] == (["k_conv_reduce"] if grid[2] > 1 else [])
+""")
