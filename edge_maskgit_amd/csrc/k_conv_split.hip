@@ -43,7 +43,6 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
     constexpr int APL = BM * KS, BPL = BN * KS;  // values per part
     constexpr int BUF = 3 * (APL + BPL);
     __shared__ __attribute__((aligned(16))) uint16_t lds[2 * BUF];
-    static_assert(2 * BUF * 2 >= BM * BN * 4, "the whole tile fits LDS (rare path of the epilogue)");
 
     const int M = a.OW * a.OH, K = a.IC * a.KW * a.KH, OC = a.OC;
     const int z = blockIdx.z;
@@ -187,46 +186,64 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
             for (int i = 0; i < I; i++) acc[j][i] += rest[j][i];
     }
     // A sum that is not finite comes from operands or products that are not, where a difference of
-    // parts is NaN: such values are summed again as they are (through LDS, to index them).
-    bool bad = false;
+    // parts is NaN: a wave that holds such sums takes its tile again on v_mfma_f32_16x16x4_f32, operands
+    // straight from memory, 16 k at a time (lane l16, lg: k 4 lg + e in MFMA e), and replaces them. A
+    // tap outside the image is no product (an infinite weight there counts nothing): each slab, one
+    // tap, is summed from zero and added where the pixel's tap is inside.
+    float nf = 0.f;                      // 0, or NaN with a sum that is not finite
 #pragma unroll
     for (int j = 0; j < J; j++)
 #pragma unroll
         for (int i = 0; i < I; i++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) bad = bad || !(fabsf(acc[j][i][e]) < INFINITY);
-    if (__syncthreads_or(bad)) {
-        // (no wave reads the operands any more; the columns are each thread's own)
-        float* T = (float*)lds + tid;
+            for (int e = 0; e < 4; e++) nf = fmaf(acc[j][i][e], 0.f, nf);
+    if (__any(nf != nf)) {
+        f32x4 sum[J][I];
+        int rw0[I], rh0[I];
 #pragma unroll
-        for (int j = 0; j < J; j++)
+        for (int i = 0; i < I; i++) {
+            const int q = min(m0 + (BM / 4) * wm + 16 * i + l16, M - 1);
+            rw0[i] = q % a.OW * a.stride - a.pad, rh0[i] = q / a.OW * a.stride - a.pad;
+#pragma unroll
+            for (int j = 0; j < J; j++) sum[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll 1
+        for (int k = kbeg; k < kend; k += 16) {
+            const int c = k % a.IC, kx = (k / a.IC) % a.KW, ky = k / a.IC / a.KW;
+            f32x4 w[J];
+            float x[I][4];
+            uint64_t in[I];
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                w[j] = *(const f32x4*)(a.wpk + (size_t)min(n0 + 64 * wn + 16 * j + l16, OC - 1) * K + k + 4 * lg);
+#pragma unroll
+            for (int i = 0; i < I; i++) {
+                const int ih = rh0[i] + ky, iw = rw0[i] + kx;
+                const bool inside = (uint32_t)ih < (uint32_t)a.IH && (uint32_t)iw < (uint32_t)a.IW;
+                in[i] = __ballot(inside);            // bits 0 .. 15: the pixels of subtile i
+                const uint32_t o = inside ? (uint32_t)(ih * a.IW + iw) * 4 + 4 * lg * plane : 0x80000000u;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    x[i][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rin, (int)o, (int)((c + e) * plane), 0));
+            }
 #pragma unroll
             for (int i = 0; i < I; i++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) T[((j * I + i) * 4 + e) * NT] = acc[j][i][e];
-#pragma unroll 1
-        for (int t = 0; t < 4 * I * J; t++) {
-            const int e = t & 3, i = (t >> 2) % I, j = (t >> 2) / I;
-            const int px = m0 + (BM / 4) * wm + 16 * i + 4 * lg + e, oc = n0 + 64 * wn + 16 * j + l16;
-            if (fabsf(T[t * NT]) < INFINITY || px >= M || oc >= OC) continue;
-            const float* x = a.in + (size_t)n * a.IC * a.IW * a.IH;
-            const float* w = a.wpk + (size_t)oc * K;
-            float v = 0.f;
-#pragma unroll 1
-            for (int k = kbeg; k < kend; k++) {
-                const int c = k % a.IC, q = k / a.IC;
-                const int ih = (px / a.OW) * a.stride - a.pad + q / a.KW, iw = (px % a.OW) * a.stride - a.pad + q % a.KW;
-                if (ih >= 0 && ih < a.IH && iw >= 0 && iw < a.IW)
-                    v = fmaf(w[k], x[((size_t)c * a.IH + ih) * a.IW + iw], v);
-            }
-            T[t * NT] = v;
+                for (int j = 0; j < J; j++) {
+                    f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][e], w[j][e], t, 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) sum[j][i][e] += (in[i] >> (4 * lg + e)) & 1 ? t[e] : 0.f;
+                }
         }
 #pragma unroll
         for (int j = 0; j < J; j++)
 #pragma unroll
             for (int i = 0; i < I; i++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) acc[j][i][e] = T[((j * I + i) * 4 + e) * NT];
+                for (int e = 0; e < 4; e++)
+                    if (!(fabsf(acc[j][i][e]) < INFINITY)) acc[j][i][e] = sum[j][i][e];
     }
     // register e of tile (i, j): pixel m0 + (BM/4) wm + 16i + 4lg + e, channel n0 + 64wn + 16j + l16
 #pragma unroll

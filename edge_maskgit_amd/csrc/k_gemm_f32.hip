@@ -130,6 +130,52 @@ __global__ __launch_bounds__(256, DB ? 2 : 4) void k_gemm_f32(GemmF32Args g) {
             products(0);
         }
     }
+    // A sum that is not finite comes from operands or products that are not, where a difference of
+    // parts is NaN: a wave that holds such sums takes its tile again on v_mfma_f32_16x16x4_f32, operands
+    // straight from memory, 16 k at a time (lane l16, lg: k 4 lg + e in MFMA e), and replaces them.
+    float nf = 0.f;                      // 0, or NaN with a sum that is not finite
+#pragma unroll
+    for (int j = 0; j < J; j++)
+#pragma unroll
+        for (int i = 0; i < I; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) nf = fmaf(acc[j][i][e], 0.f, nf);
+    if (__any(nf != nf)) {
+        f32x4 sum[J][I];
+#pragma unroll
+        for (int j = 0; j < J; j++)
+#pragma unroll
+            for (int i = 0; i < I; i++) sum[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int k0 = 0; k0 < K; k0 += KS) {
+            f32x4 w[2][I], x[2][J];
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int k = k0 + 16 * u + 4 * lg;
+#pragma unroll
+                for (int i = 0; i < I; i++) w[u][i] = *(const f32x4*)(g.w + (size_t)min(n0 + wn + 16 * i + l16, N - 1) * K + k);
+#pragma unroll
+                for (int j = 0; j < J; j++) x[u][j] = *(const f32x4*)(g.x + (size_t)min(m0 + wm + 16 * j + l16, M - 1) * K + k);
+            }
+#pragma unroll
+            for (int j = 0; j < J; j++)
+#pragma unroll
+                for (int i = 0; i < I; i++) {
+                    f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        t = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e >> 2][i][e & 3], x[e >> 2][j][e & 3], t, 0, 0, 0);
+                    sum[j][i] += t;
+                }
+        }
+#pragma unroll
+        for (int j = 0; j < J; j++)
+#pragma unroll
+            for (int i = 0; i < I; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (!(fabsf(acc[j][i][e]) < INFINITY)) acc[j][i][e] = sum[j][i][e];
+    }
     // register r of tile (i, j) is y[m0+wm+16j+l16][n0+wn+16i+4lg+r]
     // the tile leaves through LDS as whole rows, HR rows of each wave row at a time
     float* T = (float*)lds;
@@ -146,37 +192,16 @@ __global__ __launch_bounds__(256, DB ? 2 : 4) void k_gemm_f32(GemmF32Args g) {
         // thread: column tid % BN, rows tid / BN + (256 / BN) q; consecutive lanes, consecutive columns
         const int c = tid % BN, n = n0 + c;
         const float bias = g.bias && n < N ? g.bias[n] : 0.f;
-        auto row = [&](int r) { return m0 + (r / (16 * JH)) * (BM / 2) + 16 * JH * h + r % (16 * JH); };
-        auto put = [&](int m, float v) {
+#pragma unroll
+        for (int q = 0; q < HR * BN / 256; q++) {
+            const int r = tid / BN + (256 / BN) * q, m = m0 + (r / (16 * JH)) * (BM / 2) + 16 * JH * h + r % (16 * JH);
+            if (m >= M || n >= N) continue;
+            float v = T[r * TP + c];
             if (g.bias) v += bias;
             v = act_f<ACT>(v);
             const size_t o = (size_t)m * N + n;
             if (g.resid) v += g.resid[o];
             g.y[o] = v;
-        };
-        bool bad = false;
-#pragma unroll
-        for (int q = 0; q < HR * BN / 256; q++) {
-            const int r = tid / BN + (256 / BN) * q, m = row(r);
-            if (m >= M || n >= N) continue;
-            const float v = T[r * TP + c];
-            if (fabsf(v) < INFINITY) put(m, v);
-            else bad = true;
-        }
-        // A sum that is not finite comes from operands or products that are not, where a
-        // difference of parts is NaN: such values are summed again as they are (and stored once:
-        // resid may be y itself).
-        if (bad) {
-#pragma unroll 1
-            for (int q = 0; q < HR * BN / 256; q++) {
-                const int r = tid / BN + (256 / BN) * q, m = row(r);
-                if (m >= M || n >= N || fabsf(T[r * TP + c]) < INFINITY) continue;
-                const float *w = g.w + (size_t)n * K, *x = g.x + (size_t)m * K;
-                float s = 0.f;
-#pragma unroll 1
-                for (int k = 0; k < K; k++) s = fmaf(w[k], x[k], s);
-                put(m, s);
-            }
         }
     }
 }

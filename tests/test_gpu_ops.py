@@ -552,6 +552,30 @@ def test_gemm_f32_not_finite_epilogue(ctx, M, act):
     assert (np.abs(y[ok].astype(np.float64) - ref[ok]) / np.maximum(np.abs(ref[ok]).astype(np.float64), 1.0)).max() <= 2e-5
 
 
+def test_gemm_f32_not_finite_cost(ctx):
+    """rows of NaN cost at most ten times finite ones (measured: three and a half; summed one output
+    after the other 160 times)"""
+    M, N, K = 4112, 2025, 768
+    rng = np.random.default_rng(1)
+    dW, dY = ctx.upload(rng.standard_normal((N, K)).astype(np.float32)), ctx.alloc(M * N * 4)
+    ms = []
+    for fill, reps in ((1.0, 20), (np.nan, 2)):
+        dX = ctx.upload(np.full((M, K), fill, np.float32))
+        for timed in (False, True):
+            ctx.sync()
+            ctx.timer_start()
+            for _ in range(reps):
+                ctx.gemm_f32(dW, N, K, dX, M, None, 0, None, dY)
+            t = ctx.timer_stop() / reps
+        ms.append(t)
+        ctx.free(dX)
+    y = ctx.download(dY, (M, N), np.float32)
+    for b in (dW, dY):
+        ctx.free(b)
+    print(f"  finite {ms[0] * 1e3:.0f} us, NaN {ms[1] * 1e3:.0f} us")
+    assert np.isnan(y).all() and ms[1] <= 10 * ms[0]
+
+
 # ---- glue ------------------------------------------------------------------------------
 def test_get_rows_add_copy(ctx):
     print("glue ops", flush=True)
