@@ -185,8 +185,8 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
 #pragma unroll
             for (int i = 0; i < I; i++) acc[j][i] += rest[j][i];
     }
-    // A sum that is not finite comes from operands or products that are not, where a difference of
-    // parts is NaN: a wave that holds such sums takes its tile again on v_mfma_f32_16x16x4_f32, operands
+    // A sum that is not finite comes from operands or products that are not, or not in the parts' range,
+    // where a difference of parts is NaN: a wave that holds such sums takes its tile again on v_mfma_f32_16x16x4_f32, operands
     // straight from memory, 16 k at a time (lane l16, lg: k 4 lg + e in MFMA e), and replaces them. A
     // tap outside the image is no product (an infinite weight there counts nothing): each slab, one
     // tap, is summed from zero and added where the pixel's tap is inside.
@@ -196,7 +196,10 @@ __global__ __launch_bounds__(NT, 2) void k_conv2d_split(ConvPkArgs a) {
 #pragma unroll
         for (int i = 0; i < I; i++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) nf = fmaf(acc[j][i][e], 0.f, nf);
+            for (int e = 0; e < 4; e++) {
+                acc[j][i][e] *= kSplitUnscale;
+                nf = fmaf(acc[j][i][e], 0.f, nf);
+            }
     if (__any(nf != nf)) {
         f32x4 sum[J][I];
         int rw0[I], rh0[I];

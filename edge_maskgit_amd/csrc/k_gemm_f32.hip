@@ -130,8 +130,8 @@ __global__ __launch_bounds__(256, DB ? 2 : 4) void k_gemm_f32(GemmF32Args g) {
             products(0);
         }
     }
-    // A sum that is not finite comes from operands or products that are not, where a difference of
-    // parts is NaN: a wave that holds such sums takes its tile again on v_mfma_f32_16x16x4_f32, operands
+    // A sum that is not finite comes from operands or products that are not, or not in the parts' range,
+    // where a difference of parts is NaN: a wave that holds such sums takes its tile again on v_mfma_f32_16x16x4_f32, operands
     // straight from memory, 16 k at a time (lane l16, lg: k 4 lg + e in MFMA e), and replaces them.
     float nf = 0.f;                      // 0, or NaN with a sum that is not finite
 #pragma unroll
@@ -139,7 +139,10 @@ __global__ __launch_bounds__(256, DB ? 2 : 4) void k_gemm_f32(GemmF32Args g) {
 #pragma unroll
         for (int i = 0; i < I; i++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) nf = fmaf(acc[j][i][e], 0.f, nf);
+            for (int e = 0; e < 4; e++) {
+                acc[j][i][e] *= kSplitUnscale;
+                nf = fmaf(acc[j][i][e], 0.f, nf);
+            }
     if (__any(nf != nf)) {
         f32x4 sum[J][I];
 #pragma unroll

@@ -1,9 +1,18 @@
 // k_split_bf16.h — fp32 products on the bf16 matrix unit: a value is split into three bf16 parts,
 // x = hi + mid + lo, each rounded to nearest, which hold all 24 bits of its significand. Six of
-// the nine partial products reach 2^-24 of x * w and are summed; the other three (mid * lo twice,
-// lo * lo) stay below 2^-26. The running sum is rounded six times per 32 values of k, where
-// v_mfma_f32_16x16x4_f32 rounds it eight times: the result is as close to the exact sum (measured:
-// closer), at 6 x 16 against 8 x 32 cycles per 16 x 16 x 32 tile.
+// the nine partial products are summed; the other three (mid * lo twice, lo * lo) come to at most
+// 2^-24 of |x w| (|mid| <= 2^-8, |lo| <= 2^-17 of |x|; reached near x = w = 1 + 2^-8), half an ulp of
+// the product, and to far less on average. The running sum is rounded six times per 32 values of k,
+// where v_mfma_f32_16x16x4_f32 rounds it eight times: the result is as close to the exact sum
+// (measured: closer), at 6 x 16 against 8 x 32 cycles per 16 x 16 x 32 tile. (Splitting a number into
+// parts of fewer bits so that their products are exact: T. J. Dekker, A floating-point technique for
+// extending the available precision, Numer. Math. 18, 1971.)
+//
+// Range: bf16 has fp32's exponents, so the low parts of values under 2^-110 would be subnormal and lose
+// bits (6e-5 of a value of 2^-120). Values are split times 2^16 and sums taken times 2^-32, which keeps
+// every fp32 value's bits at one multiplication each (256 x 256 x 128 convolution 100 -> 101 us, 4112 x
+// 768 -> 2025 head 89 -> 92); values from 2^112 and sums from 2^96 on become infinities instead, and
+// their users redo sums that are not finite on the fp32 instruction.
 #pragma once
 #include "mgh_common.h"
 
@@ -13,12 +22,14 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32v2 __attribute__((ext_vector_type(2)));
 
+constexpr float kSplitScale = 0x1p16f, kSplitUnscale = 0x1p-32f;
+
 // eight values -> their three parts (packed pairs, element order kept)
 __device__ __forceinline__ void split_bf16(const f32x4 a, const f32x4 b, u32x4& hi, u32x4& mid, u32x4& lo) {
     const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-        float u = x[2 * p], v = x[2 * p + 1];
+        float u = x[2 * p] * kSplitScale, v = x[2 * p + 1] * kSplitScale;
         auto part = [&] {
             const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32v2{u, v}, bf16x2));
             u -= __builtin_bit_cast(float, h << 16);            // exact

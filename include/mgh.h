@@ -185,7 +185,8 @@ int mgh_flash_attn_f16in(mgh_ctx* ctx, const void* d_q16, const void* d_k16, con
  *      k_mul_mat_t and its dispatch (mg-opencl.cpp:60-94, 1429-1440).
  *      y[M][N] = act(x . w^T + bias) + resid; w [N][K], x [M][K]; K % 32 == 0, 16-byte
  *      aligned w and x. Products of the full 24-bit significands (three bf16 parts per value on
- *      the bf16 matrix unit), fp32 sums. ---- */
+ *      the bf16 matrix unit; what is left out of a product is at most 2^-24 of it) over fp32's whole
+ *      range, fp32 sums; infinities and NaN as fp32 products and sums give them. d_resid may be d_y. ---- */
 int mgh_gemm_f32(mgh_ctx* ctx, const float* d_w, int N, int K, const float* d_x, int M,
                  const float* d_bias, int act, const float* d_resid, float* d_y);
 

@@ -489,6 +489,52 @@ def test_gemm_f32_vs_float64(ctx, M, N, K, act, res):
     assert err <= 2e-6
 
 
+# exponents of x and w (ranges of powers of two): the smallest normal and subnormal numbers against
+# large ones (products and sums of ordinary size), and values past the range that the parts are scaled for
+@pytest.mark.parametrize("M", [65, 1089])
+@pytest.mark.parametrize("ex,ew", [((-126, -100), (90, 110)), ((-149, -120), (100, 111)), ((90, 110), (-126, -100)),
+                                   ((112, 126), (-126, -90)), ((-100, -64), (-40, -20)), ((40, 60), (30, 50))])
+def test_gemm_f32_whole_range(ctx, M, ex, ew):
+    """each output within 2e-6 of sum_k |w x| (as test_gemm_f32_vs_float64) or of the smallest normal
+    number, over fp32's whole exponent range"""
+    N, K = 1000, 64
+    print(f"gemm_f32 range M={M} x 2^{ex} w 2^{ew}", flush=True)
+    rng = np.random.default_rng(1000 + M + ex[0] + ew[0])
+
+    def wide(lo, hi, *shape):
+        v = rng.uniform(1, 2, shape) * rng.choice([-1.0, 1.0], shape)
+        return np.ldexp(v, rng.integers(lo, hi + 1, shape)).astype(np.float32)
+
+    x, w = wide(*ex, M, K), wide(*ew, N, K)
+    dW, dX, dY = ctx.upload(w), ctx.upload(x), ctx.alloc(M * N * 4)
+    ctx.gemm_f32(dW, N, K, dX, M, None, 0, None, dY)
+    y = ctx.download(dY, (M, N), np.float32).astype(np.float64)
+    for t in (dW, dX, dY):
+        ctx.free(t)
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    ref, mag = x @ w.T, np.abs(x) @ np.abs(w).T
+    assert mag.max() < 2.0 ** 127
+    err = float((np.abs(y - ref) / (mag + 2.0 ** -126)).max())
+    print(f"  err / sum of magnitudes {err:.2e}")
+    assert err <= 2e-6
+
+
+@pytest.mark.parametrize("v", [1 + 2.0 ** -8, 1 + 2.0 ** -8 + 2.0 ** -16, 1.0 - 2.0 ** -9])
+def test_gemm_f32_equal_operands(ctx, v):
+    """equal operands, where the products left out (at most 2^-24 of a product each) add up with one
+    sign: that and the running sum's roundings (2^-24 of it, six per 32 k, K = 128) in the worst case"""
+    M, N, K = 70, 100, 128
+    dW, dX, dY = ctx.upload(np.full((N, K), v, np.float32)), ctx.upload(np.full((M, K), v, np.float32)), ctx.alloc(M * N * 4)
+    ctx.gemm_f32(dW, N, K, dX, M, None, 0, None, dY)
+    y = ctx.download(dY, (M, N), np.float32).astype(np.float64)
+    for t in (dW, dX, dY):
+        ctx.free(t)
+    ref = K * float(np.float32(v)) ** 2
+    err = float(np.abs(y - ref).max() / ref)
+    print(f"  relative error {err:.2e}")
+    assert err <= 2.0 ** -24 * (1 + 6 * K / 32)
+
+
 @pytest.mark.parametrize("M", [70, 1100])
 def test_gemm_f32_not_finite(ctx, M):
     """infinities, NaN and values next to the largest float give what fp32 products and sums give"""

@@ -182,6 +182,38 @@ def test_conv2d_not_finite(ctx):
         assert (np.abs(y[ok] - w32[ok]) / np.maximum(1.0, np.abs(w32[ok]))).max() <= 2e-5
 
 
+@pytest.mark.parametrize("IW,IC,OC,ex,ew", [(20, 64, 24, (-126, -100), (90, 110)), (130, 32, 130, (-149, -120), (100, 111)),
+                                            (16, 512, 128, (90, 110), (-126, -100)), (20, 64, 24, (112, 120), (-126, -90))])
+def test_conv2d_whole_range(ctx, IW, IC, OC, ex, ew):
+    """3 x 3, each output within 2e-6 of the sum of its products' magnitudes (a few fp32 roundings) over
+    fp32's whole exponent range: inputs 2^ex, weights 2^ew, with and without K split, 128- and 256-pixel
+    tiles"""
+    print(f"conv2d range IW={IW} IC={IC} OC={OC} x 2^{ex} w 2^{ew}", flush=True)
+    rng = np.random.default_rng(1000 + IW + ex[0])
+
+    def wide(lo, hi, *shape):
+        v = rng.uniform(1, 2, shape) * rng.choice([-1.0, 1.0], shape)
+        return np.ldexp(v, rng.integers(lo, hi + 1, shape)).astype(np.float32)
+
+    x, ker = wide(*ex, IC, IW, IW), wide(*ew, OC, IC, 3, 3)
+    dX, dK, dY = ctx.upload(x), ctx.upload(ker), ctx.alloc(OC * IW * IW * 4)
+    ctx.conv2d(dX, IW, IW, IC, 1, dK, 3, 3, OC, 1, 1, dY)
+    y = ctx.download(dY, (OC, IW * IW), np.float32).astype(np.float64)
+    for b in (dX, dK, dY):
+        ctx.free(b)
+    xp, k64 = np.pad(x.astype(np.float64), ((0, 0), (1, 1), (1, 1))), ker.astype(np.float64)
+    ref, mag = np.zeros_like(y), np.zeros_like(y)
+    for kh in range(3):
+        for kw in range(3):
+            win = xp[:, kh:kh + IW, kw:kw + IW].reshape(IC, -1)
+            ref += k64[:, :, kh, kw] @ win
+            mag += np.abs(k64[:, :, kh, kw]) @ np.abs(win)
+    assert mag.max() < 2.0 ** 127
+    err = float((np.abs(y - ref) / (mag + 2.0 ** -126)).max())
+    print(f"  err / sum of magnitudes {err:.2e}")
+    assert err <= 2e-6
+
+
 def test_conv2d_not_finite_cost(ctx):
     """sums that are not finite are taken again with fp32 products at about the cost of an fp32
     convolution: an image of NaN costs at most ten times a finite one (measured: three; summed one
