@@ -150,3 +150,30 @@ for side, ic, oc, ksz in ((64, 48, 128, 3), (16, 48, 512, 3), (32, 80, 128, 3), 
     assert grid[2] == -(-slabs // per), (side, ic, oc, grid, per)
     assert [r[0] for r in reduce] == (["k_conv_reduce"] if grid[2] > 1 else [])
 """)
+
+
+def test_attention_route():
+    """the kernel by strides and length: whole head up to 272 keys, the long one beyond, whole head
+    again up to 512 keys for rows closer together than a head, else the one for any strides"""
+    run("""
+def route(f, S, D=48, H=3, B=2, st=None, **kw):
+    E = H * D
+    f(X, X + 0x1000, X + 0x2000, st or (1, 3 * E, D, 3 * E * S), D, S, H, B, 0.1, Y, **kw)
+    (k, n, grid), = launches()
+    return (k, int(re.findall(r"L[a-z]+([0-9]+)E", n)[1])) if k == "k_attn_head" else k
+
+close = lambda S: (1, 16, 16 * S + 48, 3 * (16 * S + 48))
+f32, f16 = c.flash_attn_f16kv, lambda *a, **kw: c.flash_attn_f16in(*a, None, (1, 144, 48, 144 * a[5]), **kw)
+for f in (f32, f16):
+    assert [route(f, S) for S in (1, 64, 65, 128, 129, 272)] == [("k_attn_head", t) for t in (4, 4, 8, 8, 17, 17)]
+    assert [route(f, S) for S in (273, 512)] == ["k_attn_long"] * 2
+    assert [route(f, S, st=close(S)) for S in (272, 273, 384, 385, 512)] == [("k_attn_head", t) for t in (17, 24, 24, 32, 32)]
+assert route(f32, 513) == route(f32, 70000) == "k_attn_long"
+assert route(f32, 513, st=close(513)) == "k_flash_attn_f16kv"
+assert route(f32, 600, st=(2, 300, 100, 300 * 600)) == route(f32, 20, st=(2, 300, 100, 6000)) == "k_flash_attn_f16kv"
+try:
+    f16(X, X + 0x1000, X + 0x2000, (1, 432, 48, 432 * 513), 48, 513, 3, 2, 0.1, Y)
+    raise SystemExit("no error")
+except ema.MghError:
+    pass
+""")

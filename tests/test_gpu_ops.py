@@ -350,6 +350,38 @@ def test_flash_attn_long_not_finite(ctx, D, S, H):
             assert np.isfinite(got).all() and np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
 
 
+# rows closer together than a head: the whole-head kernel up to 512 keys (its 17-, 24- and 32-tile
+# forms), the kernel for any strides beyond
+@pytest.mark.parametrize("D,S,R", [(48, 270, 16), (48, 300, 20), (16, 384, 8), (64, 385, 32), (32, 512, 4), (48, 500, 44), (48, 600, 16),
+                                   (32, 320, 0)])
+def test_flash_attn_overlapping_rows(ctx, D, S, R):
+    """key t's features start R elements after key t - 1's (R = 0: one key for all): against float64 on
+    the fp16-rounded operands (bar of the other attention tests), fp16 inputs equal bit for bit"""
+    H, B = 2, 2
+    print(f"flash_attn overlapping rows D={D} S={S} R={R}", flush=True)
+    rng = np.random.default_rng(D + S + R)
+    P = -(-(S * R + D) // 8) * 8                  # elements between heads
+    x = rng.standard_normal((3, B, H, P)).astype(np.float32)
+    h = np.lib.stride_tricks.sliding_window_view(x.astype(np.float16).astype(np.float64), D, axis=-1)
+    q, k, v = h[..., np.arange(S) * R, :]         # [B][H][S][D]
+    sc = q @ k.swapaxes(-1, -2) * D ** -0.5
+    p = np.exp(sc - sc.max(-1, keepdims=True))
+    ref = (p @ v / p.sum(-1, keepdims=True)).transpose(0, 2, 1, 3).reshape(B * S, H * D)
+    st, ost = (1, R, P, H * P), (1, H * D, D, H * D * S)
+    d, do = ctx.upload(x), ctx.alloc(B * S * H * D * 4)
+    n = B * H * P
+    ctx.flash_attn_f16kv(d.ptr, d.ptr + 4 * n, d.ptr + 8 * n, st, D, S, H, B, D ** -0.5, do, o_strides=ost)
+    o = ctx.download(do, (B * S, H * D), np.float32)
+    assert _rel(o, ref) <= 2e-5
+    if S <= 512:
+        d16 = ctx.upload(x.astype(np.float16))
+        ctx.flash_attn_f16in(d16.ptr, d16.ptr + 2 * n, d16.ptr + 4 * n, st, D, S, H, B, D ** -0.5, do, None, ost)
+        assert np.array_equal(ctx.download(do, (B * S, H * D), np.float32).view(np.uint32), o.view(np.uint32))
+        ctx.free(d16)
+    for t in (d, do):
+        ctx.free(t)
+
+
 def test_flash_attn_long_strides(ctx):
     """The same attention through strides the long kernel does not take (features two elements
     apart: the kernel for any strides) and through ones it takes: both within 2e-5 max|ref| of
