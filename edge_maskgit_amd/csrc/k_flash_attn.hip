@@ -1017,13 +1017,13 @@ hipError_t launch_long(const FaArgs& a, hipStream_t s) {
 }
 
 // q/k/v whose rows are features in order, spaced at least a head apart, that the staging's 8- or
-// 16-byte loads and 31-bit byte offsets can take; the workgroup count fits an int
+// 16-byte loads and 31-bit byte offsets can take; the launch's threads fit 32 bits
 bool long_ok(const FaArgs& a, int D) {
     auto al = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
     const bool ptrs = a.q16 ? al(a.q16) && al(a.k16) && al(a.v16) : al(a.q) && al(a.k) && al(a.v);
     return D % 16 == 0 && ptrs && a.st[0] == 1 && a.st[1] >= D && ((int64_t)a.S + 512) * a.st[1] * 4 < (1ll << 31) &&
            a.st[1] % 4 == 0 && a.st[2] % 4 == 0 && a.st[3] % 4 == 0 && a.scale > 0.f &&
-           (int64_t)a.H * a.B * (a.S / 32 + 1) < (1ll << 31);
+           (int64_t)a.H * a.B * (a.S / 64 + 2) * 512 < (1ll << 32);
 }
 
 bool head_ok(const FaArgs& a, int D) {

@@ -68,7 +68,9 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t lds, hipStream_t) {
     auto it = g_names.find(f);
-    if (it == g_names.end() || !g.x || !g.y || !g.z || g.y > 65535 || g.z > 65535 || b.x * b.y * b.z > 1024 || lds > 65536)
+    // (threads per dimension fit 32 bits, as the runtime requires)
+    const bool wide = (uint64_t)g.x * b.x >> 32 || (uint64_t)g.y * b.y >> 32 || (uint64_t)g.z * b.z >> 32;
+    if (it == g_names.end() || wide || !g.x || !g.y || !g.z || g.y > 65535 || g.z > 65535 || b.x * b.y * b.z > 1024 || lds > 65536)
         return ret(hipErrorInvalidConfiguration);
     g_launches.push_back(Launch{it->second, g, b, lds});
     return hipSuccess;

@@ -171,6 +171,9 @@ for f in (f32, f16):
 assert route(f32, 513) == route(f32, 70000) == "k_attn_long"
 assert route(f32, 513, st=close(513)) == "k_flash_attn_f16kv"
 assert route(f32, 600, st=(2, 300, 100, 300 * 600)) == route(f32, 20, st=(2, 300, 100, 6000)) == "k_flash_attn_f16kv"
+# more threads than a launch of the long kernel may have
+assert route(f16, 400, D=16, H=64, B=65535) == ("k_attn_head", 32)
+assert route(f32, 600, D=16, H=64, B=65535) == "k_flash_attn_f16kv"
 try:
     f16(X, X + 0x1000, X + 0x2000, (1, 432, 48, 432 * 513), 48, 513, 3, 2, 0.1, Y)
     raise SystemExit("no error")
