@@ -87,6 +87,18 @@ TRAFFIC_FILE = {"dq": "k_gemm_fc_dq", "h16": "k_gemm_fc_f16", "packed": "k_gemm_
 # bytes each path's GEMM kernel reads per weight, Q8_0 / Q4_K
 WEIGHT_BYTES = {"dq": {8: 1.0625, 12: 0.5625}, "raw": {8: 1.0625, 12: 0.5625},
                 "h16": {8: 2.0, 12: 2.0}, "packed": {8: 2.125, 12: 2.25}}
+
+
+def path_kernel(path, wtype, M):
+    """Kernel label and weight bytes per weight of a step of four FCs at M rows: Q4_K on the quantized
+    bytes is expanded to fp16 once per call at the many-row sizes (from 1025 rows all four FCs), so
+    each weight's 0.5625 bytes are read, 2 written and 2 read by the fp16 form."""
+    if path == "dq" and wtype == ema.WTYPE_Q4_K and M >= 1025:
+        return {"kernel": "k_expand_q4 + k_gemm_fc<..., WQ=0>", "weight_bytes_read": 0.5625 + 2.0,
+                "weight_bytes_written": 2.0}
+    return {"kernel": KERNEL[path], "weight_bytes_read": WEIGHT_BYTES[path][wtype]}
+
+
 PATH_NAME = {"packed": "int8_dot", "raw": "int8_dot_raw", "h16": "dequant_f16", "dq": "dequant_q"}
 WORKLOAD_PATH = {
     "h16": "dequantize-fused path (weights dequantized once to fp16 at upload; per FC one GEMM "
@@ -97,8 +109,9 @@ WORKLOAD_PATH = {
     "raw": "int8-dot path on GGUF blocks as stored",
     "dq": "dequantize-fused path on the quantized bytes (per FC one GEMM launch reading the Q8_0 / "
           "Q4_K blocks, regrouped once at upload into MFMA fragment order at the GGUF byte count, "
-          "decoded to fp16 in registers inside the K loop; fp32 activations rounded to fp16 as they "
-          "are read; fp16 MFMA with fp32 accumulation; fused epilogue)"}
+          "decoded to fp16 in registers inside the K loop, Q4_K with many rows once per call into fp16 "
+          "scratch; fp32 activations rounded to fp16 as they are read; fp16 MFMA with fp32 "
+          "accumulation; fused epilogue)"}
 ALGO = {"packed": 1, "raw": 1, "h16": 2, "dq": 2}
 
 
@@ -817,12 +830,12 @@ def main():
                 st = max(10, a.steps // 2) if mm > 1025 else a.steps
                 sm, sg, _ = measure(ctx, mm, wt, st, a.warmup, a.rotate_gb, use_graphs=a.graphs, path=pth)
                 ent[PATH_NAME[pth]] = {
-                    "kernel": KERNEL[pth], "weight_bytes_read": WEIGHT_BYTES[pth][wt],
+                    **path_kernel(pth, wt, mm),
                     "ms_per_step": round(sm, 5), "tops": round(layer_ops(mm) / (sm * 1e-3) / 1e12, 2),
                     "gemm_tops": round(layer_ops(mm) / (sg * 1e-3) / 1e12, 2),
                     "frac_of_hbm_roofline": round(ab / (HBM_PEAK_GBS * 1e9) / (sm * 1e-3), 4)}
             if (mm, wt) == (M, wtype):
-                ent[PATH_NAME[a.path]] = {"kernel": KERNEL[a.path], "weight_bytes_read": WEIGHT_BYTES[a.path][wt],
+                ent[PATH_NAME[a.path]] = {**path_kernel(a.path, wt, mm),
                                           "ms_per_step": round(ms_step, 5), "tops": round(value, 2),
                                           "gemm_tops": round(ops / (ms_gemms * 1e-3) / 1e12, 2),
                                           "frac_of_hbm_roofline": extra["step_frac_of_hbm_roofline"],

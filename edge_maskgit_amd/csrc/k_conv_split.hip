@@ -4,15 +4,15 @@
 //
 // What bounds it: v_mfma_f32_16x16x4_f32 runs at 1/16 of the bf16 rate, so six bf16 products cost
 // 96 cycles where the fp32 instruction costs 256 (16 x 16 x 32 values). The splitting is VALU work
-// (5.5 operations per value), so a tile should use each split value often: 256 pixels x 128 channels
+// (6.5 operations per value), so a tile should use each split value often: 256 pixels x 128 channels
 // per workgroup of 8 waves (64 x 64 each), one workgroup per CU and two waves per SIMD. Per 32-deep
-// K step a wave issues 96 MFMAs (1536 cycles) and splits 24 values per lane (132 operations, 528
+// K step a wave issues 96 MFMAs (1536 cycles) and splits 24 values per lane (156 operations, 624
 // cycles) for the next step, interleaved with the MFMAs. 128-pixel tiles (32 x 64 per wave) where
 // the larger ones leave CUs idle.
-// Measured: 256 x 256 x 128, one image 177 -> 95 us (203 TFLOP/s of conv work; MFMA busy 53%, the
-// rest LDS latency and VALU that the two waves per SIMD do not cover), error against 64 bits 3.1e-7
-// -> 2.7e-7. The small products in accumulators of their own: 1.1e-7 but 98 us (64 registers more,
-// so fragments are read just before use); the six of a step summed from zero: 7e-8 but 108 us (64
+// Measured: 256 x 256 x 128, one image 177 -> 98 us (197 TFLOP/s of conv work; MFMA busy 47%, VALU 35%,
+// the rest LDS latency that the two waves per SIMD do not cover), error against 64 bits 3.1e-7 ->
+// 2.7e-7. The small products in accumulators of their own: 1.1e-7 but 3 us more (64 registers more,
+// so fragments are read just before use); the six of a step summed from zero: 7e-8 but 13 us more (64
 // additions per step). With K split, where a workgroup per CU and its latency set the time, the
 // accumulators of their own cost nothing and are taken (128 x 128 x 128, two images: 66 us either way,
 // 7.9e-8 against 1.9e-7).
@@ -278,8 +278,9 @@ void launch_conv_split(const ConvPkArgs& a, hipStream_t s) {
     // 256-pixel tiles while they give most CUs a workgroup, else 128-pixel ones (3 x 3, us, 256 / 128
     // pixels: 256 x 256 x 128 95 / 110, 64 x 64 x 256 40 / 45, 16 x 16 x 512 in 32 splits with two
     // images 32 / 35; with one image, 128 large workgroups, 33 / 25; 32 x 32 x 256 27 / 24; the 1 x 1
-    // 128 x 128 x 128, 64 large workgroups, 22 / 14). Both add each output's K range in the same
-    // order, so the choice, which depends on the batch, does not change a result.
+    // 128 x 128 x 128, 64 large workgroups, 22 / 14; all before the values were scaled, at most 3%
+    // each). Both add each output's K range in the same order, so the choice, which depends on the
+    // batch, does not change a result.
     const int64_t wgs = (int64_t)((a.OW * a.OH + 255) / 256) * ((a.OC + BN - 1) / BN) * a.N * a.splits;
     if (wgs >= 200) launch_split_t<256>(a, s);
     else launch_split_t<128>(a, s);

@@ -553,7 +553,7 @@ hipError_t launch_head(const FaArgs& a, hipStream_t s) {
 // block with a single wave's queries is split over the keys instead, each wave reading its own
 // fragments from memory without the staging or its barriers.
 // Measured (16 heads, D = 48, one image) against the kernel for any strides: S = 1025 114 -> 18 us,
-// S = 4097 549 -> 122 us (16-bit MFMA work at full rate: ~50 us, VALU ~55 us), error against
+// S = 4097 549 -> 122 us (VALU busy 62 us of it, the matrix unit 42), error against
 // 64 bits 3.8e-7 -> 2.1e-7 and 6.6e-7 -> 2.8e-7.
 constexpr int LKT = 64;                  // keys per chunk
 constexpr int LVLD = LKT + 8;            // V^T row stride (halves): 9 16-byte slots

@@ -9,9 +9,10 @@
 // gfx950 mapping: fp32 products on the bf16 matrix unit, every value split into three bf16 parts as
 // it goes into LDS (k_split_bf16.h): v_mfma_f32_16x16x4_f32 runs at 1/16 of the bf16 rate, and six
 // bf16 products cost 96 cycles where it costs 256. 64 x 64 output tiles per 256-thread workgroup
-// (2 x 2 waves of 2 x 2 MFMA tiles), K in steps of 32. What bounds it now is the splitting (5.5 VALU
-// operations per value of w and x in every tile) beside the MFMAs. The 768 -> 2025 head against the
-// fp32 instruction on the same tiles: M = 257 22.3 -> 19.2 us, M = 4112 123 -> 90 us; error against
+// (2 x 2 waves of 2 x 2 MFMA tiles), K in steps of 32. What bounds it now is the splitting (6.5 VALU
+// operations per value of w and x in every tile) beside the MFMAs: at M = 4112 the VALU is busy 49% of
+// the time, the matrix unit 34%. The 768 -> 2025 head against the fp32 instruction on the same tiles:
+// M = 257 22.3 -> 19.9 us, M = 4112 123 -> 92 us; error against
 // 64 bits 5.0e-7 -> 4.2e-7. Weights take the MFMA A role so a lane holds four consecutive output
 // columns of one row; the tile leaves through LDS in whole rows (N = 2025: no aligned stores).
 #include "mgh_common.h"
@@ -224,7 +225,8 @@ hipError_t launch_gemm_f32(const GemmF32Args& a, hipStream_t s) {
     if (a.M == 0) return hipSuccess;
     // up to one workgroup per CU the K loop's latency counts (M = 257: 19.2 against 23.1 us), beyond
     // it the number of workgroups that share a CU (M = 514: 24.6 against 25.6; M = 4112: 90 against
-    // 102). 128-row tiles in either direction: 92 us and more at M = 4112, 33 at M = 514.
+    // 102). 128-row tiles in either direction: 92 us and more at M = 4112, 33 at M = 514. (All before
+    // the values were scaled, which adds 3-4% to each.)
     const int64_t tiles = (int64_t)((a.N + TB - 1) / TB) * ((a.M + TB - 1) / TB);
     return tiles <= 256 ? launch_t<true>(a, s) : launch_t<false>(a, s);
 }

@@ -230,8 +230,9 @@ __global__ __launch_bounds__(256, 2) void k_conv2d_pkn(ConvPkArgs a) {
 // neighbouring pixels of every channel from the 3 x 6 inputs of one input channel (three 16-byte
 // and six 4-byte buffer loads, taps outside the image past the range), the weights broadcast from
 // LDS; the 8 waves of a workgroup take IC / 8 input channels each for the same 256 pixels, and their
-// partial sums are added in wave order. 108 FMAs per channel and lane bound it (256 x 256 x 128 -> 3:
-// 6.3 us of VALU; measured 48 -> 18 us per image).
+// partial sums are added in wave order. 256 x 256 x 128 -> 3: 6.3 us of VALU (108 FMAs per channel and
+// lane) behind the latency of its loads; measured one image 46.7 -> 24.6 us, two 100 -> 41, of eight 18
+// each.
 template <int OCN>
 __global__ __launch_bounds__(512) void k_conv2d_out(ConvPkArgs a) {
     constexpr int WP = OCN * 9 + (4 - OCN * 9 % 4) % 4;      // floats per input channel, whole 16 bytes
