@@ -526,16 +526,17 @@ hipError_t launch_head(const FaArgs& a, hipStream_t s) {
 }
 
 // Long sequences (S > 272): online softmax over 64-key chunks, a wave holding QT 16-query tiles
-// (each K / V fragment read from LDS serves QT tiles), QG waves side by side along the queries
-// and KS key groups of QG waves that take every KS-th chunk; the key groups' (max, sum, O) are
-// merged through LDS at the end. The work is VALU-bound (4.5 operations per score, one of them
-// a quarter-rate exp2), so:
+// (each K / V fragment read from LDS serves QT tiles) and QG waves side by side along the queries.
+// The keys go to KS * SEQ groups, group g taking every KS * SEQ-th chunk from the g-th on: KS groups of
+// QG waves side by side, or SEQ groups one after the other in the same waves; the groups' (max,
+// sum, O) are merged through LDS, in both cases alike. The VALU is the busiest unit (4.5 operations per
+// score, one of them a quarter-rate exp2), so:
 //  * the products, the row sums from the matrix unit and the transposed P . V are k_attn_head's,
 //    as is P = hi + lo but for the rounding: both parts to nearest (v_cvt_pk_f16_f32, as fast as the
-//    truncating form), at most 1.2e-7 of P lost against 3.6e-7; one 32-deep MFMA covers 32 features / keys, whose order inside a
-//    fragment is free as long as both operands share it, so K rows (padded with zeros to 32) and
-//    V^T rows (keys permuted within 32: position 8 lg + 4 (t % 2) + r holds key 16 (t % 2) + 4 lg
-//    + r) are read with one conflict-free 16-byte read per fragment;
+//    truncating form), at most 1.2e-7 of P lost against 3.6e-7; one 32-deep MFMA covers 32 features /
+//    keys, whose order inside a fragment is free as long as both operands share it, so K rows
+//    (padded with zeros to 32) and V^T rows (keys permuted within 32: position 8 lg + 4 (t % 2) + r
+//    holds key 16 (t % 2) + 4 lg + r) are read with one conflict-free 16-byte read per fragment;
 //  * the softmax reference of a query only has to be near its maximum: it starts 7 below the
 //    first chunk's (log2 units), so p = 2^7 there, and moves (and O is rescaled) only when a score
 //    of the wave exceeds it by more than 15, a wave-uniform branch almost never taken after the
@@ -550,8 +551,8 @@ hipError_t launch_head(const FaArgs& a, hipStream_t s) {
 // while it computes the current one, rounds once and stores fp16 to the other LDS buffer, V as
 // 4 x 4 blocks transposed in registers: one barrier per chunk.
 // A sequence of 2^k + 1 tokens (the class token) leaves one query past the whole blocks: a last
-// block with a single wave's queries is split over the keys instead, each wave reading its own
-// fragments from memory without the staging or its barriers.
+// block with a single wave's queries is split over the keys instead (NV parts, each wave reading its
+// own fragments from memory without the staging or its barriers).
 // Measured (16 heads, D = 48, one image) against the kernel for any strides: S = 1025 114 -> 18 us,
 // S = 4097 549 -> 122 us (VALU busy 62 us of it, the matrix unit 42), error against
 // 64 bits 3.8e-7 -> 2.1e-7 and 6.6e-7 -> 2.8e-7.
@@ -999,7 +1000,7 @@ void launch_long_t(const FaArgs& a, hipStream_t s) {
 //    4 46.9 / 44.0, 1025 x 16 186 / 149; D = 64: 513 x 8 44.7 / 33.2. Side by side while its 64-query
 //    blocks run in one round (two per CU; D = 64: one), or while the 128-query blocks' last round is so
 //    empty that they take longer (a CU's round of two waves per SIMD: 1.5 times as long; 1300 x 3: 50 /
-//    62). With one group instead, whose sums are others, a batch took up to 15% less (1025 x 4: 38.8): the
+//    62). With one group instead, whose sums are others, a batch took up to 20% less (1025 x 4: 38.8): the
 //    first group's state costs LDS and so one of three workgroups per CU.
 template <int DC>
 hipError_t launch_long(const FaArgs& a, hipStream_t s) {
