@@ -845,7 +845,8 @@ __global__ __launch_bounds__(64 * QG * KS) void k_attn_long(FaArgs a, int nblk, 
         if constexpr (SEQ == 1) {
             for (int it = 0; it + 1 < nit; it++) {
                 __syncthreads();         // this buffer is filled, the other one no longer read
-                if (KS == 1 || (it + 1) * KS + kg < nch) load((it + 1) * KS + kg);   // (else: the last chunk again, never read)
+                // (past the last chunk its values are stored again, never read)
+                if (KS == 1 || (it + 1) * KS + kg < nch) load((it + 1) * KS + kg);
                 if (active) step(std::false_type{}, it & 1, it * KS + kg);
                 store((it + 1) & 1);
             }
@@ -1007,7 +1008,8 @@ hipError_t launch_long(const FaArgs& a, hipStream_t s) {
     constexpr LongCut cut = kLongCut<4, 1, 2, 1>;
     const int64_t heads = (int64_t)a.H * a.B;
     const bool tail = a.S % cut.gran && a.S % cut.gran <= cut.tail;
-    const int64_t n64 = heads * ((a.S - (tail ? cut.tail : 0) + 63) / 64), n128 = heads * ((a.S - (tail ? cut.tail : 0) + 127) / 128);
+    const int body = a.S - (tail ? cut.tail : 0);        // (rounded up to blocks: the queries of whole ones)
+    const int64_t n64 = heads * ((body + 63) / 64), n128 = heads * ((body + 127) / 128);
     if ((int64_t)a.H * ((a.S + 127) / 128) >= (DC <= 3 ? 200 : 120))
         launch_long_t<DC, 4, 2, 1, 1>(a, s);
     else if (n64 + (tail ? heads : 0) <= (DC <= 3 ? 512 : 256) || 2 * ((n64 + 255) / 256) < 3 * ((n128 + 255) / 256))

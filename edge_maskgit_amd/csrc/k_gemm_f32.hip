@@ -132,8 +132,10 @@ __global__ __launch_bounds__(256, DB ? 2 : 4) void k_gemm_f32(GemmF32Args g) {
         }
     }
     // A sum that is not finite comes from operands or products that are not, or not in the parts' range,
-    // where a difference of parts is NaN: a wave that holds such sums takes its tile again on v_mfma_f32_16x16x4_f32, operands
-    // straight from memory, 16 k at a time (lane l16, lg: k 4 lg + e in MFMA e), and replaces them.
+    // where a difference of parts is NaN: a wave that holds such sums takes its tile again on
+    // v_mfma_f32_16x16x4_f32, operands straight from memory, 16 k at a time (lane l16, lg: k 4 lg + e
+    // in MFMA e), and replaces them. (4112 rows of NaN through the head: 0.30 ms; one output after the
+    // other 15.)
     float nf = 0.f;                      // 0, or NaN with a sum that is not finite
 #pragma unroll
     for (int j = 0; j < J; j++)
